@@ -13,7 +13,7 @@ CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libgale_stokes.so")
 BUILD_DIR = os.path.join(HERE, "_build")
 
-SOURCES = ["gs_kernels.hip", "gs_tile.hip", "gs_mg.hip", "gs_net.hip", "gs_learned.hip", "gs_batch.hip", "gs_weights.hip", "gs_api.hip", "gs_generate.cpp", "gs_checkpoint.cpp"]
+SOURCES = ["gs_kernels.hip", "gs_tile.hip", "gs_mg.hip", "gs_dense.hip", "gs_net.hip", "gs_learned.hip", "gs_batch.hip", "gs_weights.hip", "gs_api.hip", "gs_generate.cpp", "gs_checkpoint.cpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
@@ -48,9 +48,7 @@ def build(verbose: bool = False, jobs: int = 2) -> str:
         if p.wait() != 0:
             raise RuntimeError("hipcc failed")
     tmp = OUT + ".tmp"
-    # rocSOLVER (with rocBLAS) factors the dense coarsest multigrid operator
-    # at setup when it is too large for the host inverse
-    cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs, "-lrocsolver", "-lrocblas"]
+    cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs]
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)

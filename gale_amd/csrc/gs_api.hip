@@ -16,10 +16,10 @@
 #include <vector>
 
 #include <rocprim/device/device_radix_sort.hpp>
-#include <rocsolver/rocsolver.h>
 
 #include "../../include/gale_stokes.h"
 #include "gs_crand.h"
+#include "gs_dense.h"
 #include "gs_internal.h"
 #include "gs_learned.h"
 #include "gs_mg.h"
@@ -133,12 +133,14 @@ struct MGLevel {
   float* h32 = nullptr;
 };
 
-// Free dofs up to which the 3D hierarchy stops for a dense coarsest solve.
+// Free dofs up to which the hierarchy stops for a dense coarsest solve.
 // 96^3 coarsens 96-48-24-12 and solves the 12^3 level (5577 free dofs with
 // free-slip walls) densely: one matrix-vector product replaces the 12^3 and
-// 6^3 levels' smoothing, transfer and solve launches of every V-cycle.
+// 6^3 levels' smoothing, transfer and solve launches of every V-cycle.  A
+// mesh that is this small itself (2D up to about 53^2, 3D up to 12^3) is
+// solved directly: an inner solve is then one product with its inverse
+// instead of about 17 V-cycles of 45 small launches (32^2 sinker).
 // GALE_MG_DENSE_MAX overrides (A/B timing); at most kDenseWideMax.
-static constexpr int kDenseHostMax = 2000;  // larger inverses are formed on the device
 static int dense_max_free() {
   const char* e = std::getenv("GALE_MG_DENSE_MAX");
   int v = e ? std::atoi(e) : 6000;
@@ -152,11 +154,17 @@ struct MGData {
   int L = 0;  // index of the coarsest level
   std::vector<MGLevel> lv;
   int nfc = 0;
-  int ldk = 0;  // 0: dense inverse packed nfc x nfc; > 0: rows padded to ldk (wide solve)
+  int ldk = 0;         // row length of the dense inverse (ldk x ldk, padding the identity)
+  int dense_from = 0;  // first level whose dense inverse may be taken (raised when one is not positive definite)
   int* freeidx = nullptr;
+  int* pos = nullptr;  // row of each dof of the coarsest level in the dense inverse, -1: Dirichlet
   double* Kinv64 = nullptr;
   float* Kinv32 = nullptr;
+  double* dwork = nullptr;    // inversion scratch
+  double* pow_d = nullptr;    // per level {lambda, scale, stopped} of the power iteration, then the pivot flag
+  double* pow_h = nullptr;    // pinned copy
 };
+constexpr int kMaxLevels = 17;
 
 static void mg_free(MGData& mg);
 
@@ -174,6 +182,7 @@ struct gs_solver {
   double* hS = nullptr;
   Reducer rd{};
   double* cg_z = nullptr;
+  bool for_batch = false;  // hierarchy for the batched kernel: small coarsest level, no direct solve
   long long P_alloc = 0;  // particle count of eta / yielded
   MGData mg;
   bool setup_done = false;
@@ -1215,7 +1224,9 @@ static void mg_free(MGData& mg) {
     }
   }
   mg.lv.clear();
-  dfree(mg.freeidx); dfree(mg.Kinv64); dfree(mg.Kinv32);
+  dfree(mg.freeidx); dfree(mg.pos); dfree(mg.Kinv64); dfree(mg.Kinv32); dfree(mg.dwork); dfree(mg.pow_d);
+  if (mg.pow_h) (void)hipHostFree(mg.pow_h);
+  mg.pow_h = nullptr;
   mg.structured = false;
   mg.L = 0;
   mg.nfc = 0;
@@ -1250,20 +1261,20 @@ static int32_t mg_structure(gs_solver* s) {
   CKS(mg_alloc_level(mg.lv.back()));
   std::vector<uint8_t> flag(pb->g.N);
   CK(hipMemcpy(flag.data(), pb->bcflag, pb->g.N, hipMemcpyDeviceToHost));
-  // 3D: coarsening stops at the first level small enough for the dense
-  // coarsest solve (dense_max_free(), 6000 free dofs): an exact solve there
-  // needs fewer inner iterations than smoothing further down, and its
-  // matrix-vector product is one wide launch where the levels below would
-  // take a dozen small ones per V-cycle (96^3: 96-48-24-12, 12^3 dense).
-  // 2D levels coarsen as far as the mesh allows (the batched solver runs each
-  // instance's dense coarsest solve inside one workgroup, where a small one
-  // is cheaper).  GALE_MG_DENSE_STOP=0 / 1 overrides (A/B timing).
+  // Coarsening stops at the first level small enough for the dense coarsest
+  // solve (dense_max_free(), 6000 free dofs), the mesh itself included: an
+  // exact solve there needs fewer inner iterations than smoothing further
+  // down, and its matrix-vector product is one wide launch where the levels
+  // below would take a dozen small ones per V-cycle (96^3: 96-48-24-12, 12^3
+  // dense).  The batched solver runs each instance's coarsest solve inside
+  // one workgroup, where a small one is cheaper: its levels go on down.
+  // GALE_MG_DENSE_STOP=0 / 1 overrides (A/B timing).
   const char* dstop = std::getenv("GALE_MG_DENSE_STOP");
-  const bool dense_stop = dstop ? std::atoi(dstop) != 0 : dim == 3;
+  const bool dense_stop = !s->for_batch && (dstop ? std::atoi(dstop) != 0 : true);
   const int dense_max = dense_max_free();
   for (int lev = 0; lev < 16; lev++) {
     const Geo& gf = mg.lv.back().g;
-    if (dense_stop && lev > 0) {
+    if (dense_stop && lev >= mg.dense_from) {
       long long nfree = 0;
       for (long long n = 0; n < gf.N; n++)
         for (int d = 0; d < dim; d++) nfree += ((flag[n] >> d) & 1u) ? 0 : 1;
@@ -1326,13 +1337,14 @@ static int32_t mg_structure(gs_solver* s) {
   if (mg.nfc <= dense_max) {
     CK(dalloc(&mg.freeidx, mg.nfc));
     CK(hipMemcpy(mg.freeidx, fidx.data(), sizeof(int) * mg.nfc, hipMemcpyHostToDevice));
-    // up to kDenseHostMax free dofs the inverse is formed on the host and
-    // stored packed; larger ones are inverted on the device and stored with
-    // padded rows for the wide solve
-    mg.ldk = mg.nfc > kDenseHostMax ? (mg.nfc + 3) & ~3 : 0;
-    const long long cols = mg.ldk > 0 ? mg.ldk : mg.nfc;
-    CK(dalloc(&mg.Kinv64, (long long)mg.nfc * cols));
-    CK(dalloc(&mg.Kinv32, (long long)mg.nfc * cols));
+    mg.ldk = dense_ld(mg.nfc);
+    std::vector<int> pos(C.n, -1);
+    for (int i = 0; i < mg.nfc; i++) pos[fidx[i]] = i;
+    CK(dalloc(&mg.pos, C.n));
+    CK(hipMemcpy(mg.pos, pos.data(), sizeof(int) * C.n, hipMemcpyHostToDevice));
+    CK(dalloc(&mg.Kinv64, (long long)mg.ldk * mg.ldk));
+    CK(dalloc(&mg.Kinv32, (long long)mg.ldk * mg.ldk));
+    CK(dalloc(&mg.dwork, dense_work_count(mg.ldk)));
   } else {
     mg.nfc = -1;  // no dense coarse solve: Chebyshev smoothing on the coarsest level
   }
@@ -1344,75 +1356,11 @@ static int32_t mg_structure(gs_solver* s) {
     const char* ev = std::getenv("GALE_MG_BOTTOM");
     mg.bottom = ev && std::atoi(ev) != 0;
   }
+  CK(dalloc(&mg.pow_d, 4 * kMaxLevels + 1));
+  if (hipHostMalloc(reinterpret_cast<void**>(&mg.pow_h), sizeof(double) * (4 * kMaxLevels + 1)) != hipSuccess)
+    return GS_E_HIP;
   mg.structured = true;
   return GS_OK;
-}
-
-// In-place inverse of an SPD matrix by Cholesky (host, coarsest level only).
-// Inverse of the SPD n x n matrix held column-major in A (leading dimension
-// ld) on the device: Cholesky factor and inverse from it (rocSOLVER potrf,
-// potri on the lower triangle), then the upper triangle filled from the
-// lower.  GS_E_NAN when the matrix is not positive definite.
-static int32_t spd_inverse_device(double* A, int n, int ld, hipStream_t st) {
-  rocblas_handle h = nullptr;
-  if (rocblas_create_handle(&h) != rocblas_status_success) return GS_E_HIP;
-  int32_t ret = GS_OK;
-  rocblas_int* dinfo = nullptr;
-  rocblas_int info = 0;
-  if (rocblas_set_stream(h, st) != rocblas_status_success || hipMalloc(&dinfo, sizeof(rocblas_int)) != hipSuccess) {
-    ret = GS_E_HIP;
-  } else if (rocsolver_dpotrf(h, rocblas_fill_lower, n, A, ld, dinfo) != rocblas_status_success ||
-             hipMemcpyAsync(&info, dinfo, sizeof(info), hipMemcpyDeviceToHost, st) != hipSuccess ||
-             hipStreamSynchronize(st) != hipSuccess) {
-    ret = GS_E_HIP;
-  } else if (info != 0) {
-    ret = GS_E_NAN;
-  } else if (rocsolver_dpotri(h, rocblas_fill_lower, n, A, ld, dinfo) != rocblas_status_success ||
-             hipMemcpyAsync(&info, dinfo, sizeof(info), hipMemcpyDeviceToHost, st) != hipSuccess ||
-             hipStreamSynchronize(st) != hipSuccess) {
-    ret = GS_E_HIP;
-  } else if (info != 0) {
-    ret = GS_E_NAN;
-  } else {
-    launch_symmetrize_lower(A, n, ld, st);
-    if (hipStreamSynchronize(st) != hipSuccess) ret = GS_E_HIP;
-  }
-  if (dinfo) (void)hipFree(dinfo);
-  rocblas_destroy_handle(h);
-  return ret;
-}
-
-static bool spd_inverse(std::vector<double>& A, int n) {
-  std::vector<double> Lm(A);
-  for (int j = 0; j < n; j++) {
-    double d = Lm[(size_t)j * n + j];
-    for (int k = 0; k < j; k++) d -= Lm[(size_t)j * n + k] * Lm[(size_t)j * n + k];
-    if (!(d > 0)) return false;
-    d = std::sqrt(d);
-    Lm[(size_t)j * n + j] = d;
-    for (int i = j + 1; i < n; i++) {
-      double v = Lm[(size_t)i * n + j];
-      for (int k = 0; k < j; k++) v -= Lm[(size_t)i * n + k] * Lm[(size_t)j * n + k];
-      Lm[(size_t)i * n + j] = v / d;
-    }
-  }
-  // inverse of L, then A^-1 = L^-T L^-1
-  std::vector<double> Li((size_t)n * n, 0.0);
-  for (int c = 0; c < n; c++) {
-    for (int i = c; i < n; i++) {
-      double v = (i == c) ? 1.0 : 0.0;
-      for (int k = c; k < i; k++) v -= Lm[(size_t)i * n + k] * Li[(size_t)k * n + c];
-      Li[(size_t)i * n + c] = v / Lm[(size_t)i * n + i];
-    }
-  }
-  for (int i = 0; i < n; i++)
-    for (int j = 0; j <= i; j++) {
-      double v = 0.0;
-      for (int k = i; k < n; k++) v += Li[(size_t)k * n + i] * Li[(size_t)k * n + j];
-      A[(size_t)i * n + j] = v;
-      A[(size_t)j * n + i] = v;
-    }
-  return true;
 }
 
 // Per-setup numeric part: moments of every level, Jacobi diagonals, the
@@ -1422,7 +1370,6 @@ static int32_t mg_numeric(gs_solver* s) {
   hipStream_t st = pb->st;
   MGData& mg = s->mg;
   if (!mg.structured) CKS(mg_structure(s));
-  const int dim = pb->dim;
   launch_moments_fine(mg.lv[0].g, pb->pk, pb->off, mg.lv[0].M64, st);
   for (int l = 1; l <= mg.L; l++) launch_moments_coarsen(mg.lv[l].g, mg.lv[l - 1].g, mg.lv[l - 1].M64, mg.lv[l].M64, st);
   for (int l = 0; l <= mg.L; l++) {
@@ -1432,88 +1379,35 @@ static int32_t mg_numeric(gs_solver* s) {
     launch_make_dinv(L.diag, L.bcdof, L.dinv64, L.n, st);
     launch_d2f(L.dinv64, L.dinv32, L.n, st);
   }
-  // Chebyshev upper bound: power iteration on D^-1 K
+  // Chebyshev upper bound: 12 power iterations on D^-1 K, the normalisation
+  // on the device (one host read for all levels instead of one per iteration)
+  launch_fill(mg.pow_d, 4 * kMaxLevels + 1, 0.0, st);
   for (int l = 0; l < mg.L || (l == mg.L && mg.nfc < 0); l++) {
     MGLevel& L = mg.lv[l];
-    launch_fill(L.x, L.n, 1.0, st);
-    launch_masked_copy(L.x, L.x, L.bcdof, L.n, st);
-    double lam = 1.0;
+    launch_pow_init(L.x, L.bcdof, L.n, mg.pow_d + 4 * l, st);
     for (int it = 0; it < 12; it++) {
       launch_mom_apply<double>(L.g, L.x, L.Ax, L.M64, L.bcflag, L.h64, st);
-      // x <- D^-1 K x / |.|
-      launch_mul(L.dinv64, L.Ax, L.d, L.n, st);
-      launch_dot(L.d, L.d, L.n, s->S, S_TMP1, s->rd, st);
-      launch_dot(L.x, L.x, L.n, s->S, S_TMP2, s->rd, st);
-      CKS(read_scalars(s));
-      const double dn = std::sqrt(s->hS[S_TMP1]), xn = std::sqrt(s->hS[S_TMP2]);
-      if (!(xn > 0) || !std::isfinite(dn)) break;
-      lam = dn / xn;
-      launch_scale(L.x, L.d, 1.0 / dn, L.n, st);
+      launch_pow_step(L.x, L.Ax, L.dinv64, L.d, L.n, mg.pow_d + 4 * l, s->rd, st);
     }
-    L.lmax = lam;
   }
-  // dense coarse operator by colour probing (nodes 3 apart do not interact)
+  int* bad = reinterpret_cast<int*>(mg.pow_d + 4 * kMaxLevels);
   if (mg.nfc > 0) {
-    MGLevel& C = mg.lv[mg.L];
-    const long long N = C.g.N;
-    const int nf = mg.nfc;
-    std::vector<int> fidx(nf);
-    CK(hipMemcpy(fidx.data(), mg.freeidx, sizeof(int) * nf, hipMemcpyDeviceToHost));
-    std::vector<int> pos(C.n, -1);
-    for (int i = 0; i < nf; i++) pos[fidx[i]] = i;
-    std::vector<double> Kd((size_t)nf * nf, 0.0), v(C.n), y(C.n);
-    const int ncz = dim == 3 ? 3 : 1;
-    for (int cz = 0; cz < ncz; cz++)
-      for (int cy = 0; cy < 3; cy++)
-        for (int cx = 0; cx < 3; cx++)
-          for (int d = 0; d < dim; d++) {
-            std::fill(v.begin(), v.end(), 0.0);
-            bool any = false;
-            for (long long n = 0; n < N; n++) {
-              const long long i = n % C.g.nn[0], j = (n / C.g.nn[0]) % C.g.nn[1], k = n / (C.g.nn[0] * C.g.nn[1]);
-              if (i % 3 == cx && j % 3 == cy && k % 3 == cz && pos[n * dim + d] >= 0) {
-                v[n * dim + d] = 1.0;
-                any = true;
-              }
-            }
-            if (!any) continue;
-            CK(hipMemcpyAsync(C.x, v.data(), sizeof(double) * C.n, hipMemcpyHostToDevice, st));
-            launch_mom_apply<double>(C.g, C.x, C.Ax, C.M64, C.bcflag, C.h64, st);
-            CK(hipMemcpyAsync(y.data(), C.Ax, sizeof(double) * C.n, hipMemcpyDeviceToHost, st));
-            CK(hipStreamSynchronize(st));
-            for (long long n = 0; n < N; n++) {
-              if (v[n * dim + d] == 0.0) continue;
-              const int col = pos[n * dim + d];
-              const long long i = n % C.g.nn[0], j = (n / C.g.nn[0]) % C.g.nn[1], k = n / (C.g.nn[0] * C.g.nn[1]);
-              for (long long kk = k - 1; kk <= k + 1; kk++)
-                for (long long jj = j - 1; jj <= j + 1; jj++)
-                  for (long long ii = i - 1; ii <= i + 1; ii++) {
-                    if (ii < 0 || jj < 0 || kk < 0 || ii >= C.g.nn[0] || jj >= C.g.nn[1] || kk >= C.g.nn[2]) continue;
-                    const long long m = ii + C.g.nn[0] * (jj + C.g.nn[1] * kk);
-                    for (int d2 = 0; d2 < dim; d2++) {
-                      const int row = pos[m * dim + d2];
-                      if (row >= 0) Kd[(size_t)row * nf + col] = y[m * dim + d2];
-                    }
-                  }
-            }
-          }
-    if (mg.ldk == 0) {
-      if (!spd_inverse(Kd, nf)) return GS_E_NAN;
-      std::vector<float> Kf(Kd.begin(), Kd.end());
-      CK(hipMemcpyAsync(mg.Kinv64, Kd.data(), sizeof(double) * Kd.size(), hipMemcpyHostToDevice, st));
-      CK(hipMemcpyAsync(mg.Kinv32, Kf.data(), sizeof(float) * Kf.size(), hipMemcpyHostToDevice, st));
-      CK(hipStreamSynchronize(st));
-    } else {
-      // Kd is symmetric, so its row-major layout is also the column-major
-      // matrix; padded rows (ld = mg.ldk), padding zero
-      const int ld = mg.ldk;
-      launch_fill(mg.Kinv64, (long long)nf * ld, 0.0, st);
-      CK(hipMemcpy2DAsync(mg.Kinv64, sizeof(double) * ld, Kd.data(), sizeof(double) * nf, sizeof(double) * nf, nf,
-                          hipMemcpyHostToDevice, st));
-      CKS(spd_inverse_device(mg.Kinv64, nf, ld, st));
-      launch_d2f(mg.Kinv64, mg.Kinv32, (long long)nf * ld, st);
-      CK(hipStreamSynchronize(st));
-    }
+    const MGLevel& C = mg.lv[mg.L];
+    launch_dense_assemble(C.g, C.M64, mg.pos, mg.nfc, mg.ldk, mg.Kinv64, st);
+    launch_spd_inverse(mg.Kinv64, mg.Kinv32, mg.ldk, mg.dwork, bad, st);
+  }
+  CK(hipMemcpyAsync(mg.pow_h, mg.pow_d, sizeof(double) * (4 * kMaxLevels + 1), hipMemcpyDeviceToHost, st));
+  CK(hipStreamSynchronize(st));
+  for (int l = 0; l < mg.L || (l == mg.L && mg.nfc < 0); l++) mg.lv[l].lmax = mg.pow_h[4 * l];
+  int hbad = 0;
+  std::memcpy(&hbad, mg.pow_h + 4 * kMaxLevels, sizeof(int));
+  if (mg.nfc > 0 && hbad) {
+    // not positive definite to rounding on this level: the next coarser one
+    // is tried, down to the smallest the mesh allows
+    const int L = mg.L;
+    mg.dense_from = L + 1;
+    CKS(mg_structure(s));
+    return mg.L > L ? mg_numeric(s) : GS_E_NAN;
   }
   return GS_OK;
 }
@@ -1579,6 +1473,7 @@ static bool vcycle_bottom(gs_solver* s, int l) {
   a.nu = l == 0 ? s->up.mg_smooth : s->up.mg_smooth_coarse;
   a.Kinv = mg.nfc > 0 ? (sizeof(T) == 8 ? (const T*)(void*)mg.Kinv64 : (const T*)(void*)mg.Kinv32) : nullptr;
   a.freeidx = mg.freeidx;
+  a.ldk = mg.ldk;
   a.nfc = mg.nfc > 0 ? mg.nfc : 0;
   mg_bottom3(a, s->pb->st);
   return true;
@@ -1597,7 +1492,7 @@ static T* vcycle(gs_solver* s, int l) {
   if (l == mg.L) {
     if (mg.nfc > 0) {
       launch_dense_solve<T>(sizeof(T) == 8 ? (const T*)(void*)mg.Kinv64 : (const T*)(void*)mg.Kinv32, mg.freeidx,
-                            mg.nfc, mg.ldk, P.b, P.x, L.n, st);
+                            mg.pos, mg.nfc, mg.ldk, P.b, P.x, L.n, st);
       return P.x;
     }
     return cheb_smooth<T>(L, 8, (T*)nullptr, st);
@@ -1617,7 +1512,12 @@ static T* vcycle(gs_solver* s, int l) {
 static void mg_precond(gs_solver* s, const double* r, double* z) {
   MGLevel& L = s->mg.lv[0];
   hipStream_t st = s->pb->st;
-  if (s->up.precision == GS_PREC_MIXED) {
+  if (s->mg.L == 0 && s->mg.nfc > 0) {
+    // the whole mesh is solved directly, in FP64 also in the mixed mode:
+    // without a smoother an inverse rounded to FP32 stops preconditioning
+    // once the condition number passes 1e7
+    launch_dense_solve<double>(s->mg.Kinv64, s->mg.freeidx, s->mg.pos, s->mg.nfc, s->mg.ldk, r, z, L.n, st);
+  } else if (s->up.precision == GS_PREC_MIXED) {
     launch_d2f(r, L.bf, L.n, st);
     const float* x = vcycle<float>(s, 0);
     launch_f2d(x, z, L.n, st);
@@ -1687,11 +1587,14 @@ struct BatchLevelInfo {
   int nx, ny;
   double lmax;
 };
+void batch_mark(gs_solver* s);
 int32_t batch_mg_info(gs_solver* s, int* nlev, BatchLevelInfo* lv, int max_levels, int* nfc);
 int32_t batch_copy_fine(gs_solver* s, double* f, double* dinv, double* Qinv, double* M64, hipStream_t st);
 int32_t batch_copy_level(gs_solver* s, int l, float* M32, float* dinv32, uint8_t* bcflag, hipStream_t st);
 int32_t batch_copy_dense(gs_solver* s, float* Kinv32, int* freeidx, hipStream_t st);
 }  // namespace gs
+
+void gs::batch_mark(gs_solver* s) { s->for_batch = true; }
 
 int32_t gs::batch_mg_info(gs_solver* s, int* nlev, BatchLevelInfo* lv, int max_levels, int* nfc) {
   if (!s || !s->setup_done || !s->mg.structured || s->pb->dim != 2) return GS_E_INVALID;
@@ -1723,9 +1626,9 @@ int32_t gs::batch_copy_level(gs_solver* s, int l, float* M32, float* dinv32, uin
 
 int32_t gs::batch_copy_dense(gs_solver* s, float* Kinv32, int* freeidx, hipStream_t st) {
   const int nf = s->mg.nfc;
-  if (s->mg.ldk != 0) return GS_E_INVALID;  // the batched solver takes packed inverses only
   if (nf <= 0) return GS_OK;
-  CK(hipMemcpyAsync(Kinv32, s->mg.Kinv32, sizeof(float) * nf * nf, hipMemcpyDeviceToDevice, st));
+  CK(hipMemcpy2DAsync(Kinv32, sizeof(float) * nf, s->mg.Kinv32, sizeof(float) * s->mg.ldk, sizeof(float) * nf, nf,
+                      hipMemcpyDeviceToDevice, st));
   CK(hipMemcpyAsync(freeidx, s->mg.freeidx, sizeof(int) * nf, hipMemcpyDeviceToDevice, st));
   return GS_OK;
 }

@@ -32,6 +32,7 @@ struct BatchLevelInfo {
   int nx, ny;
   double lmax;
 };
+void batch_mark(gs_solver* s);
 int32_t batch_mg_info(gs_solver* s, int* nlev, BatchLevelInfo* lv, int max_levels, int* nfc);
 int32_t batch_copy_fine(gs_solver* s, double* f, double* dinv, double* Qinv, double* M64, hipStream_t st);
 int32_t batch_copy_level(gs_solver* s, int l, float* M32, float* dinv32, uint8_t* bcflag, hipStream_t st);
@@ -832,6 +833,7 @@ extern "C" int32_t gs_batch_create(int32_t count, const gs_problem_desc* descs, 
     int32_t s = gs_problem_create(&d, &pbs[i]);
     if (s != GS_OK) return fail(s);
     if ((s = gs_solver_create(pbs[i], &up, &svs[i])) != GS_OK) return fail(s);
+    batch_mark(svs[i]);
     if ((s = gs_solver_setup(svs[i], nullptr, nullptr, 0)) != GS_OK) return fail(s);
     int nl = 0, nfc = 0;
     if ((s = batch_mg_info(svs[i], &nl, info[i].data(), kMaxLev, &nfc)) != GS_OK) return fail(s);

@@ -14,6 +14,7 @@
 // Chebyshev-Jacobi, and the coarsest level is solved with a dense inverse.
 #include "gs_internal.h"
 #include "gs_mg.h"
+#include "gs_reduce.h"
 #include "gs_tile.h"
 
 #include <math.h>
@@ -405,26 +406,16 @@ void launch_resid(const T* b, const T* Ax, T* r, long long n, hipStream_t st) {
 template void launch_resid<double>(const double*, const double*, double*, long long, hipStream_t);
 template void launch_resid<float>(const float*, const float*, float*, long long, hipStream_t);
 
-// Dense coarse solve: x[free[i]] = sum_j Kinv[i][j] b[free[j]], one wavefront per row.
-template <typename T>
-__global__ void k_dense_solve(const T* __restrict__ Kinv, const int* __restrict__ freeidx, int nf, const T* __restrict__ b,
-                              T* __restrict__ x) {
-  const int row = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= nf) return;
-  T s = 0;
-  for (int j = lane; j < nf; j += 64) s += Kinv[(long long)row * nf + j] * b[freeidx[j]];
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
-  if (lane == 0) x[freeidx[row]] = s;
-}
-// Wide form: 16 rows per 1024-thread workgroup, one wavefront per row; the
-// gathered right-hand side b[free[j]] is read once per workgroup into LDS,
-// and each row is read with 16-byte loads (rows padded to ld, a multiple of
-// 4 values, so every row starts 16-byte aligned).
+// Dense coarse solve: x[free[i]] = sum_j Kinv[i][j] b[free[j]], zero on the
+// Dirichlet dofs.  16 rows per 1024-thread workgroup, one wavefront per row;
+// the gathered right-hand side b[free[j]] is read once per workgroup into
+// LDS, and each row is read with 16-byte loads (rows padded to ld, so every
+// row starts 16-byte aligned).
 template <typename T>
 __global__ __launch_bounds__(1024) void k_dense_solve_wide(const T* __restrict__ Kinv, int ld,
-                                                           const int* __restrict__ freeidx, int nf,
-                                                           const T* __restrict__ b, T* __restrict__ x) {
+                                                           const int* __restrict__ freeidx,
+                                                           const int* __restrict__ pos, int nf,
+                                                           const T* __restrict__ b, T* __restrict__ x, long long n) {
   constexpr int E = 16 / (int)sizeof(T);
   typedef T vec_t __attribute__((ext_vector_type(E)));
   __shared__ __align__(16) T sb[kDenseWideMax];
@@ -438,6 +429,8 @@ __global__ __launch_bounds__(1024) void k_dense_solve_wide(const T* __restrict__
   vec_t vn = {};
   if (live && lane * E < nf) vn = r[lane];
   for (int j = threadIdx.x; j < nf; j += blockDim.x) sb[j] = b[freeidx[j]];
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+    if (pos[i] < 0) x[i] = 0;
   __syncthreads();
   if (!live) return;
   T s = 0;
@@ -453,33 +446,63 @@ __global__ __launch_bounds__(1024) void k_dense_solve_wide(const T* __restrict__
 }
 
 template <typename T>
-void launch_dense_solve(const T* Kinv, const int* freeidx, int nf, int ld, const T* b, T* x, long long n,
-                        hipStream_t st) {
-  unsigned gb = gridn(n);
-  if (gb > 8192) gb = 8192;
-  hipLaunchKernelGGL(k_fill_mg<T>, dim3(gb), dim3(kBlock), 0, st, x, n, (T)0);
-  if (nf <= 0) return;
-  if (ld > 0)
-    hipLaunchKernelGGL(k_dense_solve_wide<T>, dim3((nf + 15) / 16), dim3(1024), 0, st, Kinv, ld, freeidx, nf, b, x);
-  else
-    hipLaunchKernelGGL(k_dense_solve<T>, dim3((nf + 3) / 4), dim3(kBlock), 0, st, Kinv, freeidx, nf, b, x);
+void launch_dense_solve(const T* Kinv, const int* freeidx, const int* pos, int nf, int ld, const T* b, T* x,
+                        long long n, hipStream_t st) {
+  hipLaunchKernelGGL(k_dense_solve_wide<T>, dim3(nf > 0 ? (nf + 15) / 16 : 1), dim3(1024), 0, st, Kinv, ld, freeidx,
+                     pos, nf, b, x, n);
 }
-template void launch_dense_solve<double>(const double*, const int*, int, int, const double*, double*, long long,
-                                         hipStream_t);
-template void launch_dense_solve<float>(const float*, const int*, int, int, const float*, float*, long long,
-                                        hipStream_t);
+template void launch_dense_solve<double>(const double*, const int*, const int*, int, int, const double*, double*,
+                                         long long, hipStream_t);
+template void launch_dense_solve<float>(const float*, const int*, const int*, int, int, const float*, float*,
+                                        long long, hipStream_t);
 
-__global__ void k_symmetrize_lower(double* __restrict__ A, int n, int ld) {
-  const long long nn = (long long)n * n;
-  for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < nn; t += (long long)gridDim.x * blockDim.x) {
-    const int i = (int)(t % n), j = (int)(t / n);
-    if (i < j) A[i + (long long)j * ld] = A[j + (long long)i * ld];
-  }
+// Power iteration on D^-1 K: x = 1 on the free dofs, then per step
+// d = D^-1 (K x), lambda = |d| / |x|, x = d / |d|.  st4 = {lambda, 1 / |d|,
+// stopped}; a step whose norms are zero or not finite stops the iteration
+// with the last lambda.
+__global__ void k_pow_init(double* __restrict__ x, const uint8_t* __restrict__ bc, long long n, double* st4) {
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+    x[i] = bc[i] ? 0.0 : 1.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) st4[0] = 1.0;
 }
-void launch_symmetrize_lower(double* A, int n, int ld, hipStream_t st) {
-  unsigned gb = gridn((long long)n * n);
-  if (gb > 65536) gb = 65536;
-  hipLaunchKernelGGL(k_symmetrize_lower, dim3(gb), dim3(kBlock), 0, st, A, n, ld);
+__global__ void k_pow_dots(const double* __restrict__ x, const double* __restrict__ Ax,
+                           const double* __restrict__ dinv, double* __restrict__ d, long long n, Reducer rd) {
+  double v[2] = {0.0, 0.0};
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
+    const double di = dinv[i] * Ax[i], xi = x[i];
+    d[i] = di;
+    v[0] += di * di;
+    v[1] += xi * xi;
+  }
+  block_partials<2, false>(v, rd);
+}
+struct OpPow {
+  double* st4;
+  __device__ void operator()(const double* t) const {
+    if (st4[2] != 0.0) return;
+    const double dn = sqrt(t[0]), xn = sqrt(t[1]);
+    if (!(xn > 0) || !isfinite(dn)) {
+      st4[2] = 1.0;
+      return;
+    }
+    st4[0] = dn / xn;
+    st4[1] = 1.0 / dn;
+  }
+};
+__global__ void k_pow_scale(double* __restrict__ x, const double* __restrict__ d, long long n, const double* st4) {
+  const double sc = st4[1];
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+    x[i] = sc * d[i];
+}
+void launch_pow_init(double* x, const uint8_t* bc, long long n, double* st4, hipStream_t st) {
+  hipLaunchKernelGGL(k_pow_init, dim3(grid_for(n)), dim3(kBlock), 0, st, x, bc, n, st4);
+}
+void launch_pow_step(double* x, const double* Ax, const double* dinv, double* d, long long n, double* st4, Reducer rd,
+                     hipStream_t st) {
+  const int nb = reduce_grid(n);
+  hipLaunchKernelGGL(k_pow_dots, dim3(nb), dim3(kBlock), 0, st, x, Ax, dinv, d, n, rd);
+  reduce_finish<2, false>(rd, nb, OpPow{st4}, st);
+  hipLaunchKernelGGL(k_pow_scale, dim3(grid_for(n)), dim3(kBlock), 0, st, x, d, n, st4);
 }
 
 }  // namespace gs

@@ -55,8 +55,9 @@ struct BotArgs {
   BotLevel<T> lv[kBotMaxLevels];
   int nlev;              // lv[nlev - 1] is the coarsest level
   int nu;                // Chebyshev steps per smoothing
-  const T* Kinv;         // dense coarsest inverse (nfc x nfc), or nullptr
+  const T* Kinv;         // dense coarsest inverse (rows of ldk values), or nullptr
   const int* freeidx;
+  int ldk;
   int nfc;               // 0: eight Chebyshev steps on the coarsest level
 };
 // A level fits the bottom kernel when its node accumulator fits in 64 KiB of LDS.
@@ -101,6 +102,9 @@ __host__ __device__ inline long long mom_index(const Geo& g, int k, long long e)
   if (k < G * (27 / G)) return base + (long long)G * (k / G) * kTileThreads + G * local + k % G;
   return base + (long long)k * kTileThreads + local;
 }
+// Adds every element's matrix to the lower triangle of A (row-major, ld): one
+// thread per element column, pos[dof] the row of a dof or -1.
+void launch_dense_elements(const Geo& g, const double* Mom, const int* pos, int ld, double* A, hipStream_t st);
 // Halo buffer length (values) for one apply on this mesh.
 long long tile_halo_size(const Geo& g);
 

@@ -761,6 +761,68 @@ void tile_apply_moments_epi(const Geo& g, const float* x, float* y, float* halo,
 }
 
 // ---------------------------------------------------------------------------
+// Dense operator of a coarsest level
+// ---------------------------------------------------------------------------
+// Column `col` of element matrix e is the element's force for a unit nodal
+// value.  The elements go in 2^dim parity colours (no two of a colour share a
+// node), so each entry is added without conflicts and in a fixed order.
+template <int DIM>
+__global__ void k_dense_elements(Geo g, int c, long long total, const double* __restrict__ Mom,
+                                 const int* __restrict__ pos, int ld, double* __restrict__ A) {
+  constexpr int NEN = 1 << DIM, NC = NEN * DIM;
+  const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  if (t >= total) return;
+  const long long el = t / NC;
+  const int col = (int)(t - el * NC);
+  const long long mx = (g.res[0] - (c & 1) + 1) / 2, my = (g.res[1] - ((c >> 1) & 1) + 1) / 2;
+  const int gi = (int)(2 * (el % mx) + (c & 1)), gj = (int)(2 * ((el / mx) % my) + ((c >> 1) & 1)),
+            gk = DIM == 3 ? (int)(2 * (el / (mx * my)) + ((c >> 2) & 1)) : 0;
+  const long long sy = g.nn[0], sz = g.nn[0] * g.nn[1];
+  const long long n0 = gi + sy * gj + sz * gk;
+  const int a0 = col / DIM, c0 = col % DIM;
+  const int pc = pos[(n0 + (a0 & 1) + sy * ((a0 >> 1) & 1) + sz * ((a0 >> 2) & 1)) * DIM + c0];
+  if (pc < 0) return;
+  double ye[NEN][DIM], u[NEN][DIM];
+#pragma unroll
+  for (int a = 0; a < NEN; a++)
+#pragma unroll
+    for (int d = 0; d < DIM; d++) u[a][d] = a == a0 && d == c0 ? 1.0 : 0.0;
+  if constexpr (DIM == 3) {
+    const double ix = 0.25 / (vcoord_t(g, 0, gi + 1) - vcoord_t(g, 0, gi));
+    const double iy = 0.25 / (vcoord_t(g, 1, gj + 1) - vcoord_t(g, 1, gj));
+    const double iz = 0.25 / (vcoord_t(g, 2, gk + 1) - vcoord_t(g, 2, gk));
+    double P[3][4], Q[3][4], R[3][4], M[27], m[30];
+    grad_coeffs3(u, ix, iy, iz, P, Q, R);
+    load_moments3(g, Mom, gi, gj, gk, M);
+    element_moments3(P, Q, R, M, m);
+    epilogue3(m, ix, iy, iz, ye);
+  } else {
+    const double ix = 0.5 / (vcoord_t(g, 0, gi + 1) - vcoord_t(g, 0, gi));
+    const double iy = 0.5 / (vcoord_t(g, 1, gj + 1) - vcoord_t(g, 1, gj));
+    element2(u, ix, iy, 0, Mom, g.E, gi + (long long)g.res[0] * gj, (const double4*)nullptr, 0, 0, ye);
+  }
+#pragma unroll
+  for (int a = 0; a < NEN; a++)
+#pragma unroll
+    for (int d = 0; d < DIM; d++) {
+      const int pr = pos[(n0 + (a & 1) + sy * ((a >> 1) & 1) + sz * ((a >> 2) & 1)) * DIM + d];
+      if (pr >= pc) A[(long long)pr * ld + pc] += ye[a][d];
+    }
+}
+
+void launch_dense_elements(const Geo& g, const double* Mom, const int* pos, int ld, double* A, hipStream_t st) {
+  for (int c = 0; c < (g.dim == 3 ? 8 : 4); c++) {
+    const long long total = colour_count(g, c) * (g.dim == 3 ? 24 : 8);
+    if (total <= 0) continue;
+    const dim3 nb((unsigned)((total + kBlock - 1) / kBlock));
+    if (g.dim == 3)
+      hipLaunchKernelGGL(k_dense_elements<3>, nb, dim3(kBlock), 0, st, g, c, total, Mom, pos, ld, A);
+    else
+      hipLaunchKernelGGL(k_dense_elements<2>, nb, dim3(kBlock), 0, st, g, c, total, Mom, pos, ld, A);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Single-workgroup bottom of the 3D V-cycle
 // ---------------------------------------------------------------------------
 namespace {
@@ -939,7 +1001,7 @@ __global__ __launch_bounds__(BS) void k_mg_bottom3(BotArgs<T> a) {
       const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
       for (int row = w; row < a.nfc; row += BS / 64) {
         double s = 0;
-        for (int j = lane; j < a.nfc; j += 64) s += (double)(a.Kinv[(long long)row * a.nfc + j] * L.b[a.freeidx[j]]);
+        for (int j = lane; j < a.nfc; j += 64) s += (double)(a.Kinv[(long long)row * a.ldk + j] * L.b[a.freeidx[j]]);
         s = wave_sum_bot(s);
         if (lane == 0) L.x[a.freeidx[row]] = (T)s;
       }
