@@ -1267,18 +1267,25 @@ static int32_t mg_structure(gs_solver* s) {
   // down, and its matrix-vector product is one wide launch where the levels
   // below would take a dozen small ones per V-cycle (96^3: 96-48-24-12, 12^3
   // dense).  The batched solver runs each instance's coarsest solve inside
-  // one workgroup, where a small one is cheaper: its levels go on down.
+  // one workgroup, which reads the inverse from L2 at one compute unit's
+  // rate: there it stops at 200 free dofs (10^2 with free-slip walls, 0.16
+  // MB), below at least one smoothed level (its V-cycle is FP32 throughout);
+  // 32 sinkers of 16^2 to 48^2, four seeds: 794 ms against 954 with levels
+  // down to 2 elements a side.  300 dofs (12^2) take 631 ms, but there the
+  // solution of a 24^2 instance was twice as far from the converged one.
   // GALE_MG_DENSE_STOP=0 / 1 overrides (A/B timing).
   const char* dstop = std::getenv("GALE_MG_DENSE_STOP");
-  const bool dense_stop = !s->for_batch && (dstop ? std::atoi(dstop) != 0 : true);
+  const bool dense_stop = dstop ? std::atoi(dstop) != 0 : true;
   const int dense_max = dense_max_free();
+  const int stop_max = s->for_batch ? 200 : dense_max;
+  const int stop_from = s->for_batch ? std::max(1, mg.dense_from) : mg.dense_from;
   for (int lev = 0; lev < 16; lev++) {
     const Geo& gf = mg.lv.back().g;
-    if (dense_stop && lev >= mg.dense_from) {
+    if (dense_stop && lev >= stop_from) {
       long long nfree = 0;
       for (long long n = 0; n < gf.N; n++)
         for (int d = 0; d < dim; d++) nfree += ((flag[n] >> d) & 1u) ? 0 : 1;
-      if (nfree <= dense_max) break;
+      if (nfree <= stop_max) break;
     }
     bool ok = true;
     for (int d = 0; d < dim; d++) ok = ok && gf.res[d] % 2 == 0 && gf.res[d] / 2 >= 2;
@@ -1589,8 +1596,9 @@ struct BatchLevelInfo {
 };
 void batch_mark(gs_solver* s);
 int32_t batch_mg_info(gs_solver* s, int* nlev, BatchLevelInfo* lv, int max_levels, int* nfc);
-int32_t batch_copy_fine(gs_solver* s, double* f, double* dinv, double* Qinv, double* M64, hipStream_t st);
-int32_t batch_copy_level(gs_solver* s, int l, float* M32, float* dinv32, uint8_t* bcflag, hipStream_t st);
+int32_t batch_copy_fine(gs_solver* s, double* f, double* dinv, double* Qinv, hipStream_t st);
+int32_t batch_copy_level(gs_solver* s, int l, float* dinv32, uint8_t* bcflag, hipStream_t st);
+void batch_moments(gs_solver* s, int l, const double** M64, const float** M32);
 int32_t batch_copy_dense(gs_solver* s, float* Kinv32, int* freeidx, hipStream_t st);
 }  // namespace gs
 
@@ -1606,19 +1614,21 @@ int32_t gs::batch_mg_info(gs_solver* s, int* nlev, BatchLevelInfo* lv, int max_l
   return GS_OK;
 }
 
-int32_t gs::batch_copy_fine(gs_solver* s, double* f, double* dinv, double* Qinv, double* M64, hipStream_t st) {
-  const MGLevel& L = s->mg.lv[0];
+int32_t gs::batch_copy_fine(gs_solver* s, double* f, double* dinv, double* Qinv, hipStream_t st) {
   CK(hipMemcpyAsync(f, s->f, sizeof(double) * s->n, hipMemcpyDeviceToDevice, st));
   CK(hipMemcpyAsync(dinv, s->dinv, sizeof(double) * s->n, hipMemcpyDeviceToDevice, st));
   CK(hipMemcpyAsync(Qinv, s->Qinv, sizeof(double) * s->np, hipMemcpyDeviceToDevice, st));
-  CK(hipMemcpyAsync(M64, L.M64, sizeof(double) * L.g.E * n_moments(L.g.dim), hipMemcpyDeviceToDevice, st));
   return GS_OK;
 }
 
-int32_t gs::batch_copy_level(gs_solver* s, int l, float* M32, float* dinv32, uint8_t* bcflag, hipStream_t st) {
+void gs::batch_moments(gs_solver* s, int l, const double** M64, const float** M32) {
+  *M64 = s->mg.lv[l].M64;
+  *M32 = s->mg.lv[l].M32;
+}
+
+int32_t gs::batch_copy_level(gs_solver* s, int l, float* dinv32, uint8_t* bcflag, hipStream_t st) {
   if (l < 0 || l > s->mg.L) return GS_E_INVALID;
   const MGLevel& L = s->mg.lv[l];
-  CK(hipMemcpyAsync(M32, L.M32, sizeof(float) * L.g.E * n_moments(L.g.dim), hipMemcpyDeviceToDevice, st));
   CK(hipMemcpyAsync(dinv32, L.dinv32, sizeof(float) * L.n, hipMemcpyDeviceToDevice, st));
   CK(hipMemcpyAsync(bcflag, L.bcflag, L.g.N, hipMemcpyDeviceToDevice, st));
   return GS_OK;

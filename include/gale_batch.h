@@ -59,10 +59,11 @@ typedef struct gs_batch_result {
 /* count problem descriptions (2D); each instance is set up on the device. */
 int32_t gs_batch_create(int32_t count, const gs_problem_desc* descs, gs_batch** out);
 void gs_batch_destroy(gs_batch* b);
-/* Tile shape of the batched K apply: block in {256, 512, 1024}, tile width tx
- * dividing block (tx in {16, 32, 64}). */
+/* Workgroup shape of the batched solve: block in {256, 512, 1024} threads,
+ * tx in {16, 32, 64} (one of the shapes below; shapes of one block size run
+ * alike, the stencil applies walk the nodes in order). */
 int32_t gs_batch_set_tile(gs_batch* b, int32_t block, int32_t tx);
-/* Times every tile shape on this batch (a few Uzawa iterations each, HIP
+/* Times every shape on this batch (a few Uzawa iterations each, HIP
  * events) and keeps the fastest; ms receives one time per candidate in the
  * order (256,16) (256,32) (512,32) (512,64) (1024,32) (1024,64). */
 int32_t gs_batch_autotune(gs_batch* b, const gs_batch_params* p, int32_t* block, int32_t* tx, float* ms);
