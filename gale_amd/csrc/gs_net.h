@@ -73,8 +73,11 @@ struct Work {
   uint16_t* gb = nullptr;
   uint16_t* gc = nullptr;
   uint16_t* gskip[kLevels] = {};      // gradient reaching each skip tensor through the decoder
+  uint16_t* xt = nullptr;             // channel-major padded copies of a layer's input and
+  uint16_t* gt = nullptr;             //   output gradient for its weight gradient
+  long long tmargin = 0;              // zero entries before and after their rows
   float* partial = nullptr;           // weight-gradient partial sums
-  long long partial_cap = 0;
+  float* bpart = nullptr;             // bias-gradient partial sums
   double* dpartial = nullptr;         // reductions
 };
 

@@ -19,6 +19,7 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <vector>
@@ -196,9 +197,6 @@ __global__ __launch_bounds__(256) void k_conv(const uint16_t* __restrict__ in,
   }
 }
 
-// Weight gradient: P[chunk][kk][co] = sum_{vox in chunk} X[nbr(vox,tap)][ci] * G[vox][co]
-// A = X (rows kk, K = voxels), B = G (K = voxels, columns co).  One wavefront
-// per 16-row kk tile and voxel chunk; grid (ceil(KC/4), nchunks) x 256.
 // Split-K form of k_conv for the small levels, where a wave per 16 voxels
 // leaves most of the chip idle and each wave would walk all 27 x CIN / 16 K
 // steps in sequence: S waves share one 16-voxel tile, wave w taking K steps
@@ -413,92 +411,165 @@ __global__ __launch_bounds__(256) void k_conv_tiled(const uint16_t* __restrict__
     }
 }
 
-template <int CIN, int NT>
-__global__ __launch_bounds__(256) void k_conv_wgrad(const uint16_t* __restrict__ X, const uint16_t* __restrict__ G,
-                                                    int cg, float* __restrict__ partial, int nx, int ny, int nz,
-                                                    long long BV, int chunk_len) {
-  constexpr int KT = 27 * CIN;
-  constexpr int KC = (KT + 15) / 16;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int mt = blockIdx.x * 4 + wave;
-  if (mt >= KC) return;
-  const long long c0 = (long long)blockIdx.y * chunk_len;
-  long long c1 = c0 + chunk_len;
-  if (c1 > BV) c1 = BV;
-  const int row = lane & 15, kg = lane >> 4;
-  const int kkA = mt * 16 + row;
-  const bool rowok = kkA < KT;
-  const int tap = rowok ? kkA / CIN : 0;
-  const int ci = rowok ? kkA - tap * CIN : 0;
-  const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
-  const long long V = (long long)nx * ny * nz;
-  f4 acc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; t++) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-  for (long long vb = c0; vb < c1; vb += 16) {
-    s4 a = s4{0, 0, 0, 0};
-    s4 bq[NT];
-#pragma unroll
-    for (int t = 0; t < NT; t++) bq[t] = s4{0, 0, 0, 0};
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const long long vox = vb + kg * 4 + j;
-      if (vox >= c1) continue;
-      if (rowok) {
-        long long b;
-        int x, y, z;
-        vox_xyz(vox, V, nx, ny, &b, &x, &y, &z);
-        const int xx = x + dx, yy = y + dy, zz = z + dz;
-        if (xx >= 0 && xx < nx && yy >= 0 && yy < ny && zz >= 0 && zz < nz)
-          a[j] = (short)X[(b * V + xx + (long long)nx * (yy + (long long)ny * zz)) * CIN + ci];
-      }
-#pragma unroll
-      for (int t = 0; t < NT; t++) {
-        const int co = t * 16 + row;
-        if (co < cg) bq[t][j] = (short)G[vox * cg + co];
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < NT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bq[t], acc[t], 0, 0, 0);
+// ---------------------------------------------------------------------------
+// Weight gradient
+// ---------------------------------------------------------------------------
+// dW[tap][ci][co] = sum_vox X[vox + off(tap)][ci] G[vox][co] is a matrix
+// product over voxels, so both operands are first laid out channel by channel
+// (voxels contiguous) on the grid padded by one voxel per side and with zero
+// halos: then a tap is a constant shift of the flat voxel index, no bounds are
+// tested, and a lane's eight K values are one 16-byte load.  Halo terms are
+// exact zeros (G is zero there).
+//
+// k_pad_t: out[c * stride + p] = in[vox(p)][c] for the C channels of a
+// channels-last tensor with cs stored channels; zero on the halo, up to
+// stride, and for `margin` entries after the last row (the shifted loads of
+// the last row run over into them).  A block moves kPadSub x 64 voxels through
+// LDS.  With bpart, also the block's sum of every channel: the bias gradient
+// as a by-product (one thread a channel walking 1024 voxels took 72 us a layer).
+constexpr int kPadSub = 4;
+__global__ __launch_bounds__(256) void k_pad_t(const uint16_t* __restrict__ in, int cs, int C,
+                                               uint16_t* __restrict__ out, long long stride, int margin, int nx,
+                                               int ny, int nz, int B, float* __restrict__ bpart) {
+  __shared__ __align__(16) uint16_t tile[64 * (96 + 2)];
+  __shared__ long long src[64];
+  const int ld = cs + 2, C4 = cs / 4;
+  const unsigned w = nx + 2, h = ny + 2, d = nz + 2, pv = w * h * d;
+  if (blockIdx.x == gridDim.x - 1) {  // the margin after the last row
+    for (int i = threadIdx.x; i < margin; i += 256) out[(long long)C * stride + i] = 0;
+    return;
   }
-  const int ncol = NT * 16;
-  float* P = partial + (long long)blockIdx.y * (KC * 16) * ncol;
+  float bs = 0.f;
+  for (int sub = 0; sub < kPadSub; sub++) {
+    const long long p0 = ((long long)blockIdx.x * kPadSub + sub) * 64;
+    if (p0 >= stride) break;
+    if (threadIdx.x < 64) {
+      const long long p = p0 + threadIdx.x;
+      const long long b = p / pv;
+      const unsigned q = (unsigned)(p - b * pv);
+      const int x = (int)(q % w) - 1, y = (int)((q / w) % h) - 1, z = (int)(q / (w * h)) - 1;
+      const bool in_grid = b < B && x >= 0 && x < nx && y >= 0 && y < ny && z >= 0 && z < nz;
+      src[threadIdx.x] = in_grid ? ((b * nz + z) * ny + y) * (long long)nx + x : -1;
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < 64 * C4; q += 256) {
+      const int v = q / C4, part = q - v * C4;
+      const long long sv = src[v];
+      s4 val = s4{0, 0, 0, 0};
+      if (sv >= 0) val = reinterpret_cast<const s4*>(in + sv * cs)[part];
+      uint16_t* t = tile + v * ld + part * 4;
 #pragma unroll
-  for (int t = 0; t < NT; t++)
+      for (int k = 0; k < 4; k++) t[k] = (uint16_t)val[k];
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < C * 8; q += 256) {
+      const int c = q >> 3, v0 = (q & 7) * 8;
+      s8 o;
 #pragma unroll
-    for (int i = 0; i < 4; i++) P[(long long)(mt * 16 + kg * 4 + i) * ncol + t * 16 + row] = acc[t][i];
+      for (int k = 0; k < 8; k++) o[k] = (short)tile[(v0 + k) * ld + c];
+      // stride is a multiple of 32, so whole 8-voxel pieces lie inside it
+      if (p0 + v0 < stride) *reinterpret_cast<s8*>(out + (long long)c * stride + p0 + v0) = o;
+    }
+    if (bpart && (int)threadIdx.x < C)
+      for (int v = 0; v < 64; v++) bs += bf2f(tile[v * ld + threadIdx.x]);
+    __syncthreads();
+  }
+  if (bpart && (int)threadIdx.x < C) bpart[(long long)blockIdx.x * C + threadIdx.x] = bs;
 }
 
-// grad W[kk][co] = sum over chunks (fixed order).
-__global__ void k_wgrad_reduce(const float* __restrict__ partial, int nchunk, int kt, int kcpad, int ncol, int cout,
-                               float* __restrict__ gw) {
-  const long long n = (long long)kt * cout;
+// gb[co] = sum over the blocks' partial sums, one block per channel.
+__global__ void k_bgrad_reduce(const float* __restrict__ bpart, int n, int C, float* __restrict__ gb) {
+  __shared__ float sh[kBlock / 64];
+  const int co = blockIdx.x;
+  float v = 0.f;
+  for (int k = threadIdx.x; k < n; k += blockDim.x) v += bpart[(long long)k * C + co];
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float t = 0.f;
+    for (int k = 0; k < (int)(blockDim.x >> 6); k++) t += sh[k];
+    gb[co] = t;
+  }
+}
+
+// P[group][(tap * cin + ci)][co] over the group's share of the voxels: block
+// (m tile, dy, dz) x group, its four waves a quarter of the group each, three
+// taps (dx) x NT column tiles of 16x16 accumulators a wave.  Per 32-voxel K
+// step a wave issues 3 + NT 16-byte loads for 3 NT v_mfma_f32_16x16x32_bf16,
+// the next step's in flight.  For eight 32^3 samples (the padded 16-channel
+// level is 10 MB) the 16-channel layers take 111 us, bound by the half cache
+// lines that 16 rows of 64 bytes fetch from L2, where gathering operands in
+// 2-byte loads from the channels-last tensors took 355 us; the whole backward
+// 2.4 ms (6.2 before, with the bias sums below).
+typedef s8 s8u __attribute__((aligned(2)));  // a tap's shift leaves 2-byte alignment
+template <int NT>
+__global__ __launch_bounds__(256) void k_wgrad(const uint16_t* __restrict__ X, const uint16_t* __restrict__ G,
+                                               long long stride, int cin, int cout, int w, int pl, long long kper,
+                                               float* __restrict__ partial) {
+  __shared__ f4 red[4][NT][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int mt = blockIdx.x / 9, yz = blockIdx.x - 9 * mt;
+  const int row = lane & 15, kg = lane >> 4;
+  const int off = (yz % 3 - 1) * w + (yz / 3 - 1) * pl;
+  const long long k0 = ((long long)blockIdx.y * 4 + wave) * kper;
+  const long long k1 = k0 + kper < stride ? k0 + kper : stride;
+  const uint16_t* xa = X + (long long)(mt * 16 + row) * stride + 8 * kg + off;
+  const uint16_t* gb = G + (long long)row * stride + 8 * kg;
+  f4 acc[3][NT];
+#pragma unroll
+  for (int q = 0; q < 3; q++)
+#pragma unroll
+    for (int t = 0; t < NT; t++) acc[q][t] = f4{0.f, 0.f, 0.f, 0.f};
+  s8 a[3], g[NT];
+  auto load = [&](long long k) {
+#pragma unroll
+    for (int q = 0; q < 3; q++) a[q] = *reinterpret_cast<const s8u*>(xa + k + (q - 1));
+#pragma unroll
+    for (int t = 0; t < NT; t++) g[t] = *reinterpret_cast<const s8*>(gb + (long long)t * 16 * stride + k);
+  };
+  if (k0 < k1) load(k0);
+  for (long long k = k0; k < k1; k += 32) {
+    s8 ac[3], gc[NT];
+#pragma unroll
+    for (int q = 0; q < 3; q++) ac[q] = a[q];
+#pragma unroll
+    for (int t = 0; t < NT; t++) gc[t] = g[t];
+    if (k + 32 < k1) load(k + 32);
+#pragma unroll
+    for (int q = 0; q < 3; q++)
+#pragma unroll
+      for (int t = 0; t < NT; t++) acc[q][t] = mfma_bf16(ac[q], gc[t], acc[q][t]);
+  }
+  float* P = partial + (long long)blockIdx.y * 27 * cin * cout;
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+#pragma unroll
+    for (int t = 0; t < NT; t++) red[wave][t][lane] = acc[q][t];
+    __syncthreads();
+    for (int e = threadIdx.x; e < NT * 64; e += 256) {
+      const int t = e >> 6, l = e & 63;
+      const f4 s = ((red[0][t][l] + red[1][t][l]) + red[2][t][l]) + red[3][t][l];
+      const int co = t * 16 + (l & 15), tap = yz * 3 + q;
+      if (co < cout)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int ci = mt * 16 + 4 * (l >> 4) + i;
+          if (ci < cin) P[((long long)tap * cin + ci) * cout + co] = s[i];
+        }
+    }
+    __syncthreads();
+  }
+}
+
+// grad W = sum over the groups (fixed order).
+__global__ void k_wgrad_reduce(const float* __restrict__ partial, int ngroup, long long n, float* __restrict__ gw) {
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    const int kk = (int)(i / cout), co = (int)(i % cout);
     float s = 0.f;
-    for (int c = 0; c < nchunk; c++) s += partial[((long long)c * kcpad + kk) * ncol + co];
+#pragma unroll 8
+    for (int c = 0; c < ngroup; c++) s += partial[(long long)c * n + i];
     gw[i] = s;
   }
-}
-
-// bias partials: P[chunk][co] = sum_{vox in chunk} G[vox][co]
-__global__ void k_bgrad_partial(const uint16_t* __restrict__ G, int cg, int cout, long long BV, int chunk_len,
-                                float* __restrict__ partial) {
-  const int co = threadIdx.x;
-  if (co >= cout) return;
-  const long long c0 = (long long)blockIdx.x * chunk_len;
-  long long c1 = c0 + chunk_len;
-  if (c1 > BV) c1 = BV;
-  float s = 0.f;
-  for (long long v = c0; v < c1; v++) s += bf2f(G[v * cg + co]);
-  partial[(long long)blockIdx.x * cout + co] = s;
-}
-__global__ void k_bgrad_reduce(const float* __restrict__ partial, int nchunk, int cout, float* __restrict__ gb) {
-  const int co = threadIdx.x;
-  if (co >= cout) return;
-  float s = 0.f;
-  for (int c = 0; c < nchunk; c++) s += partial[(long long)c * cout + co];
-  gb[co] = s;
 }
 
 // Weight packing.  Forward: B[kk][co] = W[kk][co].  Transposed (data
@@ -871,6 +942,9 @@ static void free_work(Work& w) {
   f(w.gb);
   f(w.gc);
   f(w.partial);
+  f(w.bpart);
+  f(w.xt);
+  f(w.gt);
   f(w.dpartial);
   w = Work{};
 }
@@ -892,7 +966,32 @@ void destroy(Net* n) {
   *n = Net{};
 }
 
-static constexpr int kChunk = 1024;  // voxels per weight-gradient partial
+// Weight-gradient layout of a layer: flat length of its padded grid (one row
+// per channel), reach of a tap's shift, groups of voxels and K values a wave.
+struct WgradPlan {
+  long long stride, kper;
+  int w, pl, ngroup, nblk;
+};
+static WgradPlan wgrad_plan(const Shape& sh, int l) {
+  const LayerSpec& L = kSpec[l];
+  const int nx = sh.nx >> L.level, ny = sh.ny >> L.level, nz = sh.nz >> L.level;
+  WgradPlan p;
+  p.w = nx + 2;
+  p.pl = (nx + 2) * (ny + 2);
+  p.stride = ((long long)sh.batch * p.pl * (nz + 2) + 31) / 32 * 32;
+  const int mt = (L.cin + 15) / 16;
+  // about a thousand blocks, but at least four K steps a wave and at most 64
+  // partial sums to add
+  long long g = 1024 / (9 * mt);
+  if (g > 64) g = 64;
+  if (g > p.stride / 512) g = p.stride / 512;
+  if (g < 1) g = 1;
+  p.kper = ((p.stride + 4 * g - 1) / (4 * g) + 31) / 32 * 32;
+  p.ngroup = (int)((p.stride + 4 * p.kper - 1) / (4 * p.kper));
+  p.nblk = (int)((p.stride + 64 * kPadSub - 1) / (64 * kPadSub));
+  return p;
+}
+static inline int wgrad_margin(const WgradPlan& p) { return p.pl + p.w + 2 + 32; }
 
 int ensure_work(Net* n, const Shape& sh) {
   if (n->work.sh == sh && n->work.x4) return GS_OK;
@@ -924,15 +1023,26 @@ int ensure_work(Net* n, const Shape& sh) {
   NCK(al(&w.ga, gmax));
   NCK(al(&w.gb, gmax));
   NCK(al(&w.gc, gmax));
-  long long pc = 0;
+  long long pc = 0, xc = 0, gc = 0, bc = 0;
+  w.tmargin = 0;
   for (int l = 0; l < kLayers; l++) {
     const LayerSpec& L = kSpec[l];
-    const long long nch = (w.BV[L.level] + kChunk - 1) / kChunk;
-    const long long c = nch * kchunks(L.cin) * 16LL * ntiles(L.cout) * 16LL;
-    pc = c > pc ? c : pc;
+    const WgradPlan p = wgrad_plan(sh, l);
+    const long long m = (wgrad_margin(p) + 31) / 32 * 32;
+    w.tmargin = m > w.tmargin ? m : w.tmargin;
+    pc = std::max(pc, (long long)p.ngroup * 27 * L.cin * L.cout);
+    xc = std::max(xc, (L.cin + 15) / 16 * 16 * p.stride);
+    gc = std::max(gc, (long long)ntiles(L.cout) * 16 * p.stride);
+    bc = std::max(bc, (long long)p.nblk * L.cout);
   }
-  w.partial_cap = pc;
+  // rows start tmargin entries in: the first row's shifted loads run below it
+  // and the last row's beyond it, both over zeros
+  NCK(al(&w.xt, xc + 2 * w.tmargin));
+  NCK(al(&w.gt, gc + 2 * w.tmargin));
+  NCK(hipMemset(w.xt, 0, sizeof(uint16_t) * (xc + 2 * w.tmargin)));
+  NCK(hipMemset(w.gt, 0, sizeof(uint16_t) * (gc + 2 * w.tmargin)));
   NCK(hipMalloc(&w.partial, sizeof(float) * pc));
+  NCK(hipMalloc(&w.bpart, sizeof(float) * bc));
   NCK(hipMalloc(&w.dpartial, sizeof(double) * 65536));
   return GS_OK;
 }
@@ -1021,20 +1131,38 @@ static int launch_conv(int cin, int nt, bool f32, const uint16_t* in, const void
   return launch_conv_kw<16>(cin, nt, f32, in, Wp, bias, out, cout_store, nx, ny, nz, BV, relu, st);
 }
 
-static int launch_wgrad(int cin, int nt, const uint16_t* X, const uint16_t* G, int cg, float* partial, int nx,
-                        int ny, int nz, long long BV, hipStream_t st) {
-  const int kc = kchunks(cin);
-  const unsigned nchunk = (unsigned)((BV + kChunk - 1) / kChunk);
-  const dim3 grid((unsigned)((kc + 3) / 4), nchunk), block(256);
-#define X(C, N)                                                                                                   \
-  if (cin == C && nt == N) {                                                                                      \
-    hipLaunchKernelGGL((k_conv_wgrad<C, N>), grid, block, 0, st, X, G, cg, partial, nx, ny, nz, BV, kChunk);      \
-    return GS_OK;                                                                                                 \
-  }
-  CONV_CASES(X)
+// dW and db of layer l from its input x and the gradient g of its output
+// (cg stored channels).
+static int launch_wgrad(Net* n, int l, const uint16_t* x, const uint16_t* g, int cg, int nx, int ny, int nz) {
+  Work& w = n->work;
+  const LayerSpec& L = kSpec[l];
+  hipStream_t st = n->st;
+  const WgradPlan p = wgrad_plan(w.sh, l);
+  const int margin = wgrad_margin(p), B = w.sh.batch;
+  uint16_t *xt = w.xt + w.tmargin, *gt = w.gt + w.tmargin;
+  hipLaunchKernelGGL(k_pad_t, dim3(p.nblk + 1), dim3(256), 0, st, x, L.cin, L.cin, xt, p.stride, margin, nx, ny, nz,
+                     B, (float*)nullptr);
+  hipLaunchKernelGGL(k_pad_t, dim3(p.nblk + 1), dim3(256), 0, st, g, cg, L.cout, gt, p.stride, margin, nx, ny, nz, B,
+                     w.bpart);
+  const dim3 grid((unsigned)((L.cin + 15) / 16 * 9), (unsigned)p.ngroup), block(256);
+  switch (ntiles(L.cout)) {
+#define X(N)                                                                                                      \
+  case N:                                                                                                         \
+    hipLaunchKernelGGL(k_wgrad<N>, grid, block, 0, st, xt, gt, p.stride, L.cin, L.cout, p.w, p.pl, p.kper,        \
+                       w.partial);                                                                                \
+    break;
+    X(1) X(2) X(3) X(4) X(6)
 #undef X
-  std::fprintf(stderr, "gale_stokes(net): no weight-gradient kernel for cin %d, %d tiles\n", cin, nt);
-  return GS_E_INVALID;
+    default:
+      std::fprintf(stderr, "gale_stokes(net): no weight-gradient kernel for %d outputs\n", L.cout);
+      return GS_E_INVALID;
+  }
+  const long long nw = 27LL * L.cin * L.cout;
+  hipLaunchKernelGGL(k_wgrad_reduce, dim3(gridn(nw)), dim3(kBlock), 0, st, w.partial, p.ngroup, nw,
+                     n->g + weight_offset(l));
+  hipLaunchKernelGGL(k_bgrad_reduce, dim3(L.cout), dim3(kBlock), 0, st, w.bpart, p.nblk, L.cout,
+                     n->g + bias_offset(l));
+  return GS_OK;
 }
 
 static int lvl_dims(const Shape& sh, int l, int* nx, int* ny, int* nz) {
@@ -1103,14 +1231,8 @@ static int bwd_layer(Net* n, int l, const uint16_t* x, const uint16_t* gpre, int
   lvl_dims(w.sh, L.level, &nx, &ny, &nz);
   const long long BV = w.BV[L.level];
   hipStream_t st = n->st;
-  const int nt = ntiles(L.cout), kc = kchunks(L.cin);
-  const int nchunk = (int)((BV + kChunk - 1) / kChunk);
-  int e = launch_wgrad(L.cin, nt, x, gpre, cg, w.partial, nx, ny, nz, BV, st);
+  int e = launch_wgrad(n, l, x, gpre, cg, nx, ny, nz);
   if (e) return e;
-  hipLaunchKernelGGL(k_wgrad_reduce, dim3(gridn(27LL * L.cin * L.cout)), dim3(kBlock), 0, st, w.partial, nchunk,
-                     27 * L.cin, kc * 16, nt * 16, L.cout, n->g + weight_offset(l));
-  hipLaunchKernelGGL(k_bgrad_partial, dim3(nchunk), dim3(128), 0, st, gpre, cg, L.cout, BV, kChunk, w.partial);
-  hipLaunchKernelGGL(k_bgrad_reduce, dim3(1), dim3(128), 0, st, w.partial, nchunk, L.cout, n->g + bias_offset(l));
   if (gin) {
     const int cin_t = L.cout < 4 ? 4 : L.cout;
     e = launch_conv(cin_t, ntiles(L.cin), false, gpre, n->wt[l], nullptr, gin, L.cin, nx, ny, nz, BV, 0, st);
