@@ -1432,7 +1432,7 @@ static LvPtr<float> lvp(MGLevel& L, float*) {
   return {L.bf, L.xf, L.xf2, L.rf, L.df, L.Axf, L.M32, L.dinv32, L.h32};
 }
 
-// Chebyshev-Jacobi smoothing of K x = b on [0.1, 1.1] lambda_max(D^-1 K).
+// Chebyshev-Jacobi smoothing of K x = b on [kChebLow, kChebHigh] lambda_max(D^-1 K).
 // Each step after the first is one K apply whose node completion performs
 // the Chebyshev update (TileEpi kind 1), writing x + d into the other of the
 // level's two x buffers.  x == nullptr starts from zero (first step without
@@ -1440,7 +1440,7 @@ static LvPtr<float> lvp(MGLevel& L, float*) {
 template <typename T>
 static T* cheb_smooth(MGLevel& L, int nu, T* x, hipStream_t st) {
   LvPtr<T> P = lvp(L, (T*)nullptr);
-  const double emax = 1.1 * L.lmax, emin = 0.1 * L.lmax;
+  const double emax = kChebHigh * L.lmax, emin = kChebLow * L.lmax;
   const double theta = 0.5 * (emax + emin), delta = 0.5 * (emax - emin), sigma = theta / delta;
   double rho_prev = 1.0 / sigma;
   int k0 = 0;

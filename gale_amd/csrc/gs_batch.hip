@@ -377,8 +377,8 @@ struct Inst {
   double *fs, *fq;
 };
 
-// Chebyshev-Jacobi smoothing on one level (FP32), window [0.1, 1.1] lmax,
-// as the single-problem smoother: zero = start from x = 0.  x starts in `x`
+// Chebyshev-Jacobi smoothing on one level (FP32), window [0.1, 1.1] lmax (in
+// 2D the lower bound makes no difference here): zero = start from x = 0.  x starts in `x`
 // (or in Lx when zero) and ping-pongs; returns the buffer that holds it.
 template <int BS>
 __device__ float* bsmooth(const BArgs& A, const BLevel& L, int nu, bool zero, float* x) {

@@ -37,6 +37,17 @@ void launch_pow_init(double* x, const uint8_t* bc, long long n, double* st4, hip
 void launch_pow_step(double* x, const double* Ax, const double* dinv, double* d, long long n, double* st4, Reducer rd,
                      hipStream_t st);
 
+// Chebyshev-Jacobi smoothing damps the part [low, high] lambda_max of the
+// spectrum of D^-1 K; lambda_max comes from 12 power iterations, which fall
+// short of it.  With low = 0.1 the polynomial grows fast above the window, so
+// an estimate 10 % short costs more than the wider window gains: inner
+// iterations per Uzawa iteration with low 0.1 / 0.15 / 0.2 / 0.25 are 20.6 /
+// 8.6 / 6.3 / 6.5 (Rayleigh-Taylor 64^3), 10.2 / - / 7.9 / - (48^3), 4.5 / 4.2
+// / 3.8 / 3.9 (random viscosity 96^3), 9.0 / 8.4 / 8.2 / 8.3 (lithosphere
+// 256 x 64); learned solves of ten 48^3 and ten 64^3 fields take 11.9 / 10.8 /
+// 10.9 s in total.
+constexpr double kChebLow = 0.2, kChebHigh = 1.1;
+
 inline int n_moments(int dim) { return dim == 2 ? 9 : 27; }
 
 }  // namespace gs

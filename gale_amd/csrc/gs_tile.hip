@@ -10,6 +10,7 @@
 // two launches, every y entry is written once (plus one read-modify-write on
 // tile faces), and the result is bitwise reproducible.
 #include "gs_internal.h"
+#include "gs_mg.h"
 #include "gs_tile.h"
 
 #include <math.h>
@@ -885,7 +886,7 @@ __device__ __forceinline__ T bot_take(const BotLevel<T>& L, T* sy, long long i) 
 template <typename T, int BS>
 __device__ T* bot_cheb(const BotLevel<T>& L, int nu, T* x, T* sy) {
   const long long n = L.g.N * 3;
-  const double emax = 1.1 * L.lmax, emin = 0.1 * L.lmax;
+  const double emax = kChebHigh * L.lmax, emin = kChebLow * L.lmax;
   const double theta = 0.5 * (emax + emin), delta = 0.5 * (emax - emin), sigma = theta / delta;
   double rho_prev = 1.0 / sigma;
   int k0 = 0;
