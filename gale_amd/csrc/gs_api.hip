@@ -131,7 +131,15 @@ struct MGLevel {
   float *bf = nullptr, *xf = nullptr, *rf = nullptr, *df = nullptr, *Axf = nullptr, *xf2 = nullptr;
   double* h64 = nullptr;  // tiled-apply halo scratch
   float* h32 = nullptr;
+  double* A64 = nullptr;  // assembled rows of a small level, in the precision of the V-cycle
+  float* A32 = nullptr;
 };
+
+// Levels whose assembled rows take at most this (in FP64: 33^3 nodes in 3D,
+// 500^2 in 2D) are smoothed from them; larger ones, whose rows would come from
+// HBM, from their moments (48^3 nodes: 228 MB against 24 MB).
+constexpr long long kStencilBytes = 72LL << 20;
+static bool assembled_level(const Geo& g) { return stencil_count(g) * 8 <= kStencilBytes; }
 
 // Free dofs up to which the hierarchy stops for a dense coarsest solve.
 // 96^3 coarsens 96-48-24-12 and solves the 12^3 level (5577 free dofs with
@@ -1217,7 +1225,7 @@ static void mg_free(MGData& mg) {
     dfree(L.M64); dfree(L.M32); dfree(L.diag); dfree(L.dinv64); dfree(L.dinv32);
     dfree(L.b); dfree(L.x); dfree(L.r); dfree(L.d); dfree(L.Ax);
     dfree(L.bf); dfree(L.xf); dfree(L.rf); dfree(L.df); dfree(L.Axf); dfree(L.h64); dfree(L.h32);
-    dfree(L.x2); dfree(L.xf2);
+    dfree(L.x2); dfree(L.xf2); dfree(L.A64); dfree(L.A32);
     if (L.own_bc) {
       dfree(L.bcflag);
       dfree(L.bcdof);
@@ -1397,6 +1405,18 @@ static int32_t mg_numeric(gs_solver* s) {
       launch_pow_step(L.x, L.Ax, L.dinv64, L.d, L.n, mg.pow_d + 4 * l, s->rd, st);
     }
   }
+  // assembled rows of the small smoothed levels, in the V-cycle's precision
+  for (int l = 0; l < mg.L || (l == mg.L && mg.nfc < 0); l++) {
+    MGLevel& L = mg.lv[l];
+    if (s->for_batch || !assembled_level(L.g)) continue;
+    if (s->up.precision == GS_PREC_MIXED) {
+      if (!L.A32) CK(dalloc(&L.A32, stencil_count(L.g)));
+      launch_stencil_build<float>(L.g, L.M64, L.bcflag, L.A32, st);
+    } else {
+      if (!L.A64) CK(dalloc(&L.A64, stencil_count(L.g)));
+      launch_stencil_build<double>(L.g, L.M64, L.bcflag, L.A64, st);
+    }
+  }
   int* bad = reinterpret_cast<int*>(mg.pow_d + 4 * kMaxLevels);
   if (mg.nfc > 0) {
     const MGLevel& C = mg.lv[mg.L];
@@ -1422,32 +1442,47 @@ static int32_t mg_numeric(gs_solver* s) {
 template <typename T>
 struct LvPtr {
   T *b, *x, *x2, *r, *d, *Ax;
-  const T *M, *dinv;
+  const T *M, *dinv, *A;
   T* h;
 };
 static LvPtr<double> lvp(MGLevel& L, double*) {
-  return {L.b, L.x, L.x2, L.r, L.d, L.Ax, L.M64, L.dinv64, L.h64};
+  return {L.b, L.x, L.x2, L.r, L.d, L.Ax, L.M64, L.dinv64, L.A64, L.h64};
 }
 static LvPtr<float> lvp(MGLevel& L, float*) {
-  return {L.bf, L.xf, L.xf2, L.rf, L.df, L.Axf, L.M32, L.dinv32, L.h32};
+  return {L.bf, L.xf, L.xf2, L.rf, L.df, L.Axf, L.M32, L.dinv32, L.A32, L.h32};
+}
+
+// Smoothing step or residual of a level from its assembled rows or moments.
+template <typename T>
+static void level_epi(MGLevel& L, const LvPtr<T>& P, const T* x, const TileEpi<T>& ep, hipStream_t st) {
+  if (P.A)
+    launch_stencil_epi<T>(L.g, P.A, x, ep, st);
+  else
+    tile_apply_moments_epi(L.g, x, P.Ax, P.h, P.M, L.bcflag, ep, st);
 }
 
 // Chebyshev-Jacobi smoothing of K x = b on [kChebLow, kChebHigh] lambda_max(D^-1 K).
 // Each step after the first is one K apply whose node completion performs
 // the Chebyshev update (TileEpi kind 1), writing x + d into the other of the
-// level's two x buffers.  x == nullptr starts from zero (first step without
-// an apply).  Returns the buffer that holds the smoothed x.
+// level's two x buffers (the last step into `out` when given).  x == nullptr
+// starts from zero: the first step needs no apply and is worked out where the
+// second (or, with nu = 1, the residual) reads it, except on the 2D tiled
+// levels.  Returns the buffer that holds the smoothed x, nullptr when nu = 1
+// left it to the residual.
 template <typename T>
-static T* cheb_smooth(MGLevel& L, int nu, T* x, hipStream_t st) {
+static T* cheb_smooth(MGLevel& L, int nu, T* x, hipStream_t st, const T* b, T* out, T* beta0) {
   LvPtr<T> P = lvp(L, (T*)nullptr);
   const double emax = kChebHigh * L.lmax, emin = kChebLow * L.lmax;
   const double theta = 0.5 * (emax + emin), delta = 0.5 * (emax - emin), sigma = theta / delta;
   double rho_prev = 1.0 / sigma;
   int k0 = 0;
+  *beta0 = (T)(1.0 / theta);
   if (!x) {
-    launch_cheb<T>(P.b, nullptr, P.dinv, P.d, P.x, L.n, (T)0, (T)(1.0 / theta), 1, st);
-    x = P.x;
     k0 = 1;
+    if (!P.A && L.g.dim == 2) {
+      x = out && nu == 1 ? out : P.x;
+      launch_cheb<T>(b, nullptr, P.dinv, P.d, x, L.n, (T)0, *beta0, 1, st);
+    }
   }
   for (int k = k0; k < nu; k++) {
     T alpha = 0, beta = (T)(1.0 / theta);
@@ -1457,9 +1492,9 @@ static T* cheb_smooth(MGLevel& L, int nu, T* x, hipStream_t st) {
       beta = (T)(2.0 * rho / delta);
       rho_prev = rho;
     }
-    T* xo = x == P.x ? P.x2 : P.x;
-    TileEpi<T> ep{1, P.b, P.dinv, P.d, xo, nullptr, alpha, beta};
-    tile_apply_moments_epi(L.g, x, P.Ax, P.h, P.M, L.bcflag, ep, st);
+    T* xo = out && k == nu - 1 ? out : (x == P.x ? P.x2 : P.x);
+    TileEpi<T> ep{1, b, P.dinv, P.d, xo, nullptr, alpha, beta, *beta0};
+    level_epi<T>(L, P, x, ep, st);
     x = xo;
   }
   return x;
@@ -1486,33 +1521,37 @@ static bool vcycle_bottom(gs_solver* s, int l) {
   return true;
 }
 
-// One V-cycle for K x = b at level l (b in the level's b buffer); returns the
-// buffer holding x.
+// One V-cycle for K x = b at level l (b in the level's b buffer, or b0);
+// returns the buffer holding x (out when given).
 template <typename T>
-static T* vcycle(gs_solver* s, int l) {
+static T* vcycle(gs_solver* s, int l, const T* b0 = nullptr, T* out = nullptr) {
   MGData& mg = s->mg;
   MGLevel& L = mg.lv[l];
   hipStream_t st = s->pb->st;
   const int nu = l == 0 ? s->up.mg_smooth : s->up.mg_smooth_coarse;
   LvPtr<T> P = lvp(L, (T*)nullptr);
-  if (vcycle_bottom<T>(s, l)) return P.x;
+  if (!b0 && vcycle_bottom<T>(s, l)) return P.x;
+  const T* b = b0 ? b0 : P.b;
+  T beta0;
   if (l == mg.L) {
     if (mg.nfc > 0) {
+      T* x = out ? out : P.x;
       launch_dense_solve<T>(sizeof(T) == 8 ? (const T*)(void*)mg.Kinv64 : (const T*)(void*)mg.Kinv32, mg.freeidx,
-                            mg.pos, mg.nfc, mg.ldk, P.b, P.x, L.n, st);
-      return P.x;
+                            mg.pos, mg.nfc, mg.ldk, b, x, L.n, st);
+      return x;
     }
-    return cheb_smooth<T>(L, 8, (T*)nullptr, st);
+    return cheb_smooth<T>(L, 8, (T*)nullptr, st, b, out, &beta0);
   }
   MGLevel& C = mg.lv[l + 1];
   LvPtr<T> Q = lvp(C, (T*)nullptr);
-  T* x = cheb_smooth<T>(L, nu, (T*)nullptr, st);
-  TileEpi<T> ep{2, P.b, nullptr, nullptr, nullptr, P.r, 0, 0};
-  tile_apply_moments_epi(L.g, x, P.Ax, P.h, P.M, L.bcflag, ep, st);  // r = b - K x
+  T* x = cheb_smooth<T>(L, nu, (T*)nullptr, st, b, (T*)nullptr, &beta0);
+  TileEpi<T> ep{2, b, P.dinv, nullptr, P.x, P.r, 0, 0, beta0};
+  level_epi<T>(L, P, x, ep, st);  // r = b - K x (x null: the first Chebyshev step, left in P.x)
+  if (!x) x = P.x;
   launch_restrict<T>(C.g, L.g, P.r, Q.b, C.bcflag, st);
   T* xc = vcycle<T>(s, l + 1);
   launch_prolong_add<T>(C.g, L.g, xc, x, L.bcflag, st);
-  return cheb_smooth<T>(L, nu, x, st);
+  return cheb_smooth<T>(L, nu, x, st, b, out, &beta0);
 }
 
 // z = M^-1 r by one V-cycle (FP64, or FP32 in the mixed-precision mode).
@@ -1523,15 +1562,13 @@ static void mg_precond(gs_solver* s, const double* r, double* z) {
     // the whole mesh is solved directly, in FP64 also in the mixed mode:
     // without a smoother an inverse rounded to FP32 stops preconditioning
     // once the condition number passes 1e7
-    launch_dense_solve<double>(s->mg.Kinv64, s->mg.freeidx, s->mg.pos, s->mg.nfc, s->mg.ldk, r, z, L.n, st);
+    vcycle<double>(s, 0, r, z);
   } else if (s->up.precision == GS_PREC_MIXED) {
     launch_d2f(r, L.bf, L.n, st);
     const float* x = vcycle<float>(s, 0);
     launch_f2d(x, z, L.n, st);
   } else {
-    (void)hipMemcpyAsync(L.b, r, sizeof(double) * L.n, hipMemcpyDeviceToDevice, st);
-    const double* x = vcycle<double>(s, 0);
-    (void)hipMemcpyAsync(z, x, sizeof(double) * L.n, hipMemcpyDeviceToDevice, st);
+    vcycle<double>(s, 0, r, z);
   }
 }
 

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "gs_internal.h"
+#include "gs_tile.h"
 
 namespace gs {
 
@@ -24,6 +25,10 @@ void launch_prolong_add(const Geo& gc, const Geo& gf, const T* xc, T* xf, const 
 template <typename T>
 void launch_cheb(const T* b, const T* Ax, const T* dinv, T* d, T* x, long long n, T alpha, T beta, int first,
                  hipStream_t st);
+// Smoothing step or residual (TileEpi kinds 1 and 2, x null included) on an
+// assembled level, one launch.
+template <typename T>
+void launch_stencil_epi(const Geo& g, const T* A, const T* x, const TileEpi<T>& ep, hipStream_t st);
 template <typename T>
 void launch_resid(const T* b, const T* Ax, T* r, long long n, hipStream_t st);
 // Dense coarsest solve x = Kinv b on the free dofs (nf at most

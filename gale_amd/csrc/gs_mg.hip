@@ -274,35 +274,53 @@ __device__ __forceinline__ void node_ijk(const Geo& g, long long n, long long& i
     k = n / (g.nn[0] * g.nn[1]);
   }
 }
-// Full-weighting restriction b_C = R r_F on the nodes of the coarse level
-// (3 x 3 (x 3) stencil, weights 1 and 1/2 per axis, in stencil order).
+// Full-weighting restriction b_C = R r_F on the coarse level (3 x 3 (x 3)
+// stencil, weights 1 and 1/2 per axis).  A thread owns a coarse dof and, in
+// 3D, one of its three fine node planes, nine loads in flight; the planes'
+// sums meet in LDS.  A coarse level is small, so it is bound by the latency of
+// the loads one thread has to wait for: 48^3 -> 24^3 in FP64 takes 3.5 us, one
+// thread per node walking all 27 nodes took 8.8.
 template <typename T, int DIM>
-__global__ void k_restrict(Geo gc, Geo gf, const T* __restrict__ rf, T* __restrict__ bc, const uint8_t* __restrict__ bcflag_c) {
-  const long long n = xcd_block_mg(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (n >= gc.N) return;
-  long long I, J, K;
-  node_ijk(gc, n, I, J, K);
-  T acc[3] = {0, 0, 0};
-  const int kz0 = DIM == 3 ? -1 : 0, kz1 = DIM == 3 ? 1 : 0;
-  for (int dz = kz0; dz <= kz1; dz++) {
-    const long long k = 2 * K + dz;
-    if (k < 0 || k >= gf.nn[2]) continue;
-    const T wz = dz == 0 ? (T)1 : (T)0.5;
-    for (int dy = -1; dy <= 1; dy++) {
-      const long long j = 2 * J + dy;
-      if (j < 0 || j >= gf.nn[1]) continue;
-      const T wy = dy == 0 ? (T)1 : (T)0.5;
-      for (int dx = -1; dx <= 1; dx++) {
-        const long long i = 2 * I + dx;
-        if (i < 0 || i >= gf.nn[0]) continue;
-        const T w = wz * wy * (dx == 0 ? (T)1 : (T)0.5);
-        const long long f = i + gf.nn[0] * (j + gf.nn[1] * k);
-        for (int d = 0; d < DIM; d++) acc[d] += w * rf[f * DIM + d];
-      }
+__global__ __launch_bounds__(DIM == 3 ? 192 : 64) void k_restrict(Geo gc, Geo gf, const T* __restrict__ rf,
+                                                                  T* __restrict__ bc,
+                                                                  const uint8_t* __restrict__ bcflag_c) {
+  __shared__ T part[DIM == 3 ? 2 : 1][64];
+  const long long nd = gc.N * DIM;
+  const long long i = xcd_block_mg(blockIdx.x, gridDim.x) * 64 + threadIdx.x;
+  const int pl = DIM == 3 ? (int)threadIdx.y : 0;
+  const bool live = i < nd;
+  T s = 0;
+  unsigned bf = 0;
+  int c = 0;
+  if (live) {
+    const long long n = i / DIM;
+    c = (int)(i - n * DIM);
+    long long I, J, K;
+    node_ijk(gc, n, I, J, K);
+    if (pl == 0 && bcflag_c) bf = bcflag_c[n];
+    const long long kk = DIM == 3 ? 2 * K + pl - 1 : 0;
+    const bool inz = kk >= 0 && kk < gf.nn[2];
+    T v[9];
+#pragma unroll
+    for (int q = 0; q < 9; q++) {
+      const long long ii = 2 * I + q % 3 - 1, jj = 2 * J + q / 3 - 1;
+      const bool in = inz && ii >= 0 && ii < gf.nn[0] && jj >= 0 && jj < gf.nn[1];
+      v[q] = in ? rf[(ii + gf.nn[0] * (jj + gf.nn[1] * kk)) * DIM + c] : (T)0;
     }
+#pragma unroll
+    for (int q = 0; q < 9; q++) s += (q % 3 == 1 ? (T)1 : (T)0.5) * (q / 3 == 1 ? (T)1 : (T)0.5) * v[q];
+    if (DIM == 3 && pl != 1) s *= (T)0.5;
   }
-  const unsigned bf = bcflag_c ? bcflag_c[n] : 0u;
-  for (int d = 0; d < DIM; d++) bc[n * DIM + d] = ((bf >> d) & 1u) ? (T)0 : acc[d];
+  if (DIM == 3) {
+    if (pl > 0) part[pl - 1][threadIdx.x] = s;
+    __syncthreads();
+    if (pl > 0 || !live) return;
+    s += part[0][threadIdx.x];
+    s += part[DIM == 3 ? 1 : 0][threadIdx.x];
+  } else if (!live) {
+    return;
+  }
+  bc[i] = ((bf >> c) & 1u) ? (T)0 : s;
 }
 
 // x_F += P x_C (Q1 interpolation) on the nodes of the fine level: the up to
@@ -351,10 +369,11 @@ __global__ void k_prolong_add(Geo gc, Geo gf, const T* __restrict__ xc, T* __res
 
 template <typename T>
 void launch_restrict(const Geo& gc, const Geo& gf, const T* rf, T* bc, const uint8_t* bcflag_c, hipStream_t st) {
+  const dim3 nb((unsigned)((gc.N * gc.dim + 63) / 64));
   if (gc.dim == 3)
-    hipLaunchKernelGGL((k_restrict<T, 3>), dim3(gridn(gc.N)), dim3(kBlock), 0, st, gc, gf, rf, bc, bcflag_c);
+    hipLaunchKernelGGL((k_restrict<T, 3>), nb, dim3(64, 3), 0, st, gc, gf, rf, bc, bcflag_c);
   else
-    hipLaunchKernelGGL((k_restrict<T, 2>), dim3(gridn(gc.N)), dim3(kBlock), 0, st, gc, gf, rf, bc, bcflag_c);
+    hipLaunchKernelGGL((k_restrict<T, 2>), nb, dim3(64), 0, st, gc, gf, rf, bc, bcflag_c);
 }
 template <typename T>
 void launch_prolong_add(const Geo& gc, const Geo& gf, const T* xc, T* xf, const uint8_t* bcflag_f, hipStream_t st) {
@@ -390,6 +409,104 @@ void launch_cheb(const T* b, const T* Ax, const T* dinv, T* d, T* x, long long n
 }
 template void launch_cheb<double>(const double*, const double*, const double*, double*, double*, long long, double, double, int, hipStream_t);
 template void launch_cheb<float>(const float*, const float*, const float*, float*, float*, long long, float, float, int, hipStream_t);
+
+// ---------------------------------------------------------------------------
+// Assembled levels
+// ---------------------------------------------------------------------------
+// A small level is bound by latency, not by bytes: the tiled apply runs 54
+// workgroups on 24^3 and needs a second launch for the tile faces.  Here a
+// thread owns a row and, in 3D, one of the three node planes (64 x 3 threads;
+// the planes' sums meet in LDS), all of its 27 (2D: 18) coefficients and
+// neighbour values loaded at once, and the update follows in the same launch.
+// At 24^3 in FP64 a smoothing step takes 5 us (apply + face completion: 15),
+// reading 30 MB of coefficients from L2 in the place of 3 MB of moments.
+template <typename T, int DIM, int KIND, bool X0>
+__global__ __launch_bounds__(DIM == 3 ? 192 : 64) void k_stencil_epi(Geo g, const T* __restrict__ A,
+                                                                     const T* __restrict__ x, TileEpi<T> ep) {
+  constexpr int NB = 9;
+  __shared__ T part[DIM == 3 ? 2 : 1][64];
+  const long long nd = g.N * DIM;
+  // rows of an XCD's blocks are contiguous, so its L2 keeps their coefficients
+  const long long i = xcd_block_mg(blockIdx.x, gridDim.x) * 64 + threadIdx.x;
+  const int pl = DIM == 3 ? (int)threadIdx.y : 0;
+  const bool live = i < nd;
+  T s = 0, bi = 0, di0 = 0, xv = 0, dv = 0;
+  if (live) {
+    const unsigned n = (unsigned)(i / DIM);
+    const unsigned nx = (unsigned)g.nn[0], ny = (unsigned)g.nn[1], q = n / nx;
+    const int li = (int)(n - q * nx), lj = (int)(q % ny), lk = (int)(q / ny);
+    if (pl == 0) {  // the row's own values travel with the coefficients
+      bi = ep.b[i];
+      if (KIND == 1 || X0) di0 = ep.dinv[i];
+      if (!X0 && KIND == 1) {
+        xv = x[i];
+        if (ep.alpha != 0) dv = ep.d[i];  // a first step does not read d: its buffer may hold anything
+      }
+    }
+    const int kz = DIM == 3 ? lk + pl - 1 : 0;
+    const bool inz = DIM == 3 ? kz >= 0 && kz < (int)g.nn[2] : true;
+    T c[NB][DIM], v[NB][DIM];
+#pragma unroll
+    for (int k = 0; k < NB; k++) {
+      const int ii = li + k % 3 - 1, jj = lj + k / 3 - 1;
+      const bool in = inz && ii >= 0 && ii < (int)nx && jj >= 0 && jj < (int)ny;
+      // outside the grid the coefficients are zero: read the row's own node
+      const long long m = in ? ii + (long long)nx * (jj + (long long)ny * kz) : (long long)n;
+#pragma unroll
+      for (int d = 0; d < DIM; d++) {
+        c[k][d] = A[((long long)(pl * NB + k) * DIM + d) * nd + i];
+        v[k][d] = X0 ? ep.beta0 * ep.dinv[m * DIM + d] * ep.b[m * DIM + d] : x[m * DIM + d];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NB; k++)
+#pragma unroll
+      for (int d = 0; d < DIM; d++) s += c[k][d] * v[k][d];
+  }
+  if (DIM == 3) {
+    if (pl > 0) part[pl - 1][threadIdx.x] = s;
+    __syncthreads();
+    if (pl > 0 || !live) return;
+    s += part[0][threadIdx.x];
+    s += part[DIM == 3 ? 1 : 0][threadIdx.x];
+  } else if (!live) {
+    return;
+  }
+  if (X0) xv = ep.beta0 * di0 * bi;
+  if (KIND == 1) {
+    const T di = ep.alpha * (X0 ? xv : dv) + ep.beta * di0 * (bi - s);
+    ep.d[i] = di;
+    ep.xout[i] = xv + di;
+  } else {
+    ep.r[i] = bi - s;
+    if (X0) ep.xout[i] = xv;
+  }
+}
+
+template <typename T, int DIM>
+static void stencil_epi(const Geo& g, const T* A, const T* x, const TileEpi<T>& ep, hipStream_t st) {
+  const dim3 nb((unsigned)((g.N * DIM + 63) / 64)), bl(64, DIM == 3 ? 3 : 1);
+  if (ep.kind == 1) {
+    if (x)
+      hipLaunchKernelGGL((k_stencil_epi<T, DIM, 1, false>), nb, bl, 0, st, g, A, x, ep);
+    else
+      hipLaunchKernelGGL((k_stencil_epi<T, DIM, 1, true>), nb, bl, 0, st, g, A, x, ep);
+  } else {
+    if (x)
+      hipLaunchKernelGGL((k_stencil_epi<T, DIM, 2, false>), nb, bl, 0, st, g, A, x, ep);
+    else
+      hipLaunchKernelGGL((k_stencil_epi<T, DIM, 2, true>), nb, bl, 0, st, g, A, x, ep);
+  }
+}
+template <typename T>
+void launch_stencil_epi(const Geo& g, const T* A, const T* x, const TileEpi<T>& ep, hipStream_t st) {
+  if (g.dim == 3)
+    stencil_epi<T, 3>(g, A, x, ep, st);
+  else
+    stencil_epi<T, 2>(g, A, x, ep, st);
+}
+template void launch_stencil_epi<double>(const Geo&, const double*, const double*, const TileEpi<double>&, hipStream_t);
+template void launch_stencil_epi<float>(const Geo&, const float*, const float*, const TileEpi<float>&, hipStream_t);
 
 // r = b - Ax
 template <typename T>

@@ -23,6 +23,9 @@ struct TileGrid {
 //   kind 2: residual  r_i = b_i - ax
 // The update runs in the node-parallel launch that completes tile-face
 // nodes; y holds the apply's partial sums.  xout must not alias x.
+// With x null the input is the first Chebyshev step from zero,
+// x_i = beta0 dinv_i b_i, worked out where it is read (no launch of its own):
+// kind 1 then takes it for d as well, kind 2 also writes it to xout.
 template <typename T>
 struct TileEpi {
   int kind;
@@ -31,8 +34,15 @@ struct TileEpi {
   T* d;
   T* xout;
   T* r;
-  T alpha, beta;
+  T alpha, beta, beta0;
 };
+
+// Assembled form of a small level: the 3^dim x dim coefficients of every row,
+// A[(k * dim + c2) * n + i] for row (dof) i, neighbour k (x fastest) and its
+// component c2; rows of Dirichlet dofs zero.
+inline long long stencil_count(const Geo& g) { return (g.dim == 3 ? 81LL * 3 : 18LL * 2) * g.N; }
+template <typename T>
+void launch_stencil_build(const Geo& g, const double* Mom, const uint8_t* bcflag, T* A, hipStream_t st);
 
 // The bottom of a 3D multigrid V-cycle (the smallest levels and the coarsest
 // solve) in one workgroup: each level's K applies accumulate into one LDS

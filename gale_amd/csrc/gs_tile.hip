@@ -68,18 +68,21 @@ __device__ __forceinline__ double wave_sum_bot(double v) {
   return v;
 }
 
-// Completes dof i with ax = (K x)_i (see TileEpi); xv = x_i.
-template <typename T, int EPI>
-__device__ __forceinline__ void epi_store(const TileEpi<T>& ep, T* __restrict__ y, long long i, T ax, T xv) {
-  if (EPI == 0) {
-    y[i] = ax;
-  } else if (EPI == 1) {
-    const T rr = ep.b[i] - ax;
-    const T di = ep.alpha * ep.d[i] + ep.beta * ep.dinv[i] * rr;
+// Completes dof i with ax = (K x)_i (see TileEpi).
+template <typename T, int EPI, bool X0>
+__device__ __forceinline__ void epi_store(const TileEpi<T>& ep, const T* __restrict__ x, long long i, T ax) {
+  const T bi = ep.b[i];
+  if (EPI == 1) {
+    const T di0 = ep.dinv[i];
+    const T xv = X0 ? ep.beta0 * di0 * bi : x[i];
+    // a first step (alpha 0) does not read d: its buffer may hold anything
+    const T dv = X0 ? xv : (ep.alpha != 0 ? ep.d[i] : (T)0);
+    const T di = ep.alpha * dv + ep.beta * di0 * (bi - ax);
     ep.d[i] = di;
     ep.xout[i] = xv + di;
   } else {
-    ep.r[i] = ep.b[i] - ax;
+    ep.r[i] = bi - ax;
+    if (X0) ep.xout[i] = ep.beta0 * ep.dinv[i] * bi;
   }
 }
 
@@ -351,7 +354,7 @@ __device__ __forceinline__ void element2(const T (&u)[4][2], T ix, T iy, int for
 // ---------------------------------------------------------------------------
 // The FP32 moment form is held to 5 waves per SIMD (86 VGPRs, no spills;
 // 118 and 4 waves unconstrained); the other forms keep the compiler's choice.
-template <typename T, int FORM>
+template <typename T, int FORM, bool X0>
 __global__ __launch_bounds__(kTileThreads)
 __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && FORM == 0 ? 5 : 1))) void
 k_tile_apply3(Geo g, TileGrid tg, const T* __restrict__ x,
@@ -359,7 +362,9 @@ k_tile_apply3(Geo g, TileGrid tg, const T* __restrict__ x,
                                                               const T* __restrict__ Mom,
                                                               const typename V4<T>::type* __restrict__ pk,
                                                               const int* __restrict__ off,
-                                                              const uint8_t* __restrict__ bcflag, int mom_nt) {
+                                                              const uint8_t* __restrict__ bcflag, int mom_nt,
+                                                              const T* __restrict__ xb,
+                                                              const T* __restrict__ xdinv, T beta0) {
   constexpr int TX = kTile3X, TY = kTile3Y, TZ = kTile3Z;
   constexpr int NBX = TX + 1, NBY = TY + 1, NBZ = TZ + 1, NB = NBX * NBY * NBZ;
   // node box, one array per component (consecutive elements hit consecutive
@@ -401,7 +406,7 @@ k_tile_apply3(Geo g, TileGrid tg, const T* __restrict__ x,
       const int lx = nd % NBX, ly = (nd / NBX) % NBY, lz = nd / (NBX * NBY);
       if (lx < nbx && ly < nby && lz < nbz) {
         const long long gn = (x0 + lx) + sy_ * (y0 + ly) + sz_ * (z0 + lz);
-        vq[it] = x[gn * 3 + c];
+        vq[it] = X0 ? beta0 * xdinv[gn * 3 + c] * xb[gn * 3 + c] : x[gn * 3 + c];
         if (bcflag) mq |= ((bcflag[gn] >> c) & 1u) << it;
       }
     }
@@ -521,7 +526,7 @@ __global__ void k_tile_face3(Geo g, TileGrid tg, T* __restrict__ y, const T* __r
 // dof i = 3 n + c), so every vector access of a wavefront is one contiguous
 // run (a thread per node with three strided accesses moved about twice the
 // bytes); blocks are remapped so each XCD works on a contiguous range.
-template <typename T, int EPI>
+template <typename T, int EPI, bool X0>
 __global__ void k_tile_halo3(Geo g, TileGrid tg, const T* __restrict__ x, T* __restrict__ y,
                              const T* __restrict__ halo, const uint8_t* __restrict__ bcflag, TileEpi<T> ep) {
   constexpr int TX = kTile3X, TY = kTile3Y, TZ = kTile3Z;
@@ -549,7 +554,6 @@ __global__ void k_tile_halo3(Geo g, TileGrid tg, const T* __restrict__ x, T* __r
   }
   const int tx = min(i / TX, tg.n[0] - 1), ty = min(j / TY, tg.n[1] - 1), tz = min(k / TZ, tg.n[2] - 1);
   const int onx = (i == tx * TX && tx > 0), ony = (j == ty * TY && ty > 0), onz = (k == tz * TZ && tz > 0);
-  if (EPI == 0 && !(onx | ony | onz)) return;
   T acc = 0;
   for (int az = 0; az <= onz; az++)
     for (int ay = 0; ay <= ony; ay++)
@@ -561,12 +565,8 @@ __global__ void k_tile_halo3(Geo g, TileGrid tg, const T* __restrict__ x, T* __r
         acc += halo[(t2 * NB + ln) * 3 + c];
       }
   const bool fixed = bcflag ? ((bcflag[n] >> c) & 1u) : false;
-  if (EPI == 0) {
-    if (!fixed) y[id] += acc;
-  } else {
-    const T ax = fixed ? (T)0 : y[id] + acc;
-    epi_store<T, EPI>(ep, y, id, ax, x[id]);
-  }
+  const T ax = fixed ? (T)0 : y[id] + acc;
+  epi_store<T, EPI, X0>(ep, x, id, ax);
 }
 
 // ---------------------------------------------------------------------------
@@ -667,7 +667,7 @@ __global__ void k_tile_halo2(Geo g, TileGrid tg, const T* __restrict__ x, T* __r
   } else {
     for (int c = 0; c < 2; c++) {
       const T ax = ((bf >> c) & 1u) ? (T)0 : y[n * 2 + c] + acc[c];
-      epi_store<T, EPI>(ep, y, n * 2 + c, ax, x[n * 2 + c]);
+      epi_store<T, EPI, false>(ep, x, n * 2 + c, ax);
     }
   }
 }
@@ -704,13 +704,23 @@ static void tile_launch(const Geo& g, const T* x, T* y, T* halo, const T* Mom, c
     // non-temporal moment loads when the moments exceed a quarter of the
     // 256 MB last-level cache (they are then streamed, not reused)
     const int nt = FORM == 0 && (double)mom_count<T>(g) * sizeof(T) > 64.0e6 ? 1 : 0;
-    hipLaunchKernelGGL((k_tile_apply3<T, FORM>), dim3((unsigned)tg.ntiles), dim3(kTileThreads), 0, st, g, tg, x,
-                       y, halo, Mom, pk, off, bcflag, nt);
-    if (EPI == 0) {
+    if constexpr (EPI == 0) {
+      hipLaunchKernelGGL((k_tile_apply3<T, FORM, false>), dim3((unsigned)tg.ntiles), dim3(kTileThreads), 0, st, g, tg,
+                         x, y, halo, Mom, pk, off, bcflag, nt, nullptr, nullptr, (T)0);
       hipLaunchKernelGGL((k_tile_face3<T>), dim3(nbn), dim3(kBlock), 0, st, g, tg, y, halo, bcflag);
     } else {
       const unsigned nbd = (unsigned)((g.N * 3 + kBlock - 1) / kBlock);
-      hipLaunchKernelGGL((k_tile_halo3<T, EPI>), dim3(nbd), dim3(kBlock), 0, st, g, tg, x, y, halo, bcflag, ep);
+      if (x) {
+        hipLaunchKernelGGL((k_tile_apply3<T, FORM, false>), dim3((unsigned)tg.ntiles), dim3(kTileThreads), 0, st, g,
+                           tg, x, y, halo, Mom, pk, off, bcflag, nt, nullptr, nullptr, (T)0);
+        hipLaunchKernelGGL((k_tile_halo3<T, EPI, false>), dim3(nbd), dim3(kBlock), 0, st, g, tg, x, y, halo, bcflag,
+                           ep);
+      } else {
+        hipLaunchKernelGGL((k_tile_apply3<T, FORM, true>), dim3((unsigned)tg.ntiles), dim3(kTileThreads), 0, st, g,
+                           tg, x, y, halo, Mom, pk, off, bcflag, nt, ep.b, ep.dinv, ep.beta0);
+        hipLaunchKernelGGL((k_tile_halo3<T, EPI, true>), dim3(nbd), dim3(kBlock), 0, st, g, tg, x, y, halo, bcflag,
+                           ep);
+      }
     }
   } else {
     hipLaunchKernelGGL((k_tile_apply2<T, FORM>), dim3((unsigned)tg.ntiles), dim3(kTileThreads), 0, st, g, tg, x,
@@ -760,6 +770,89 @@ void tile_apply_moments_epi(const Geo& g, const float* x, float* y, float* halo,
                             const uint8_t* bcflag, const TileEpi<float>& ep, hipStream_t st) {
   tile_apply_epi<float>(g, x, y, halo, Mom, bcflag, ep, st);
 }
+
+// ---------------------------------------------------------------------------
+// Assembled rows of a small level
+// ---------------------------------------------------------------------------
+// One thread per (neighbour, node): the dim x dim block coupling the node to
+// that neighbour, summed over the elements that hold both in lattice order.
+template <typename T, int DIM>
+__global__ __launch_bounds__(kBlock) void k_stencil_build(Geo g, const double* __restrict__ Mom, const uint8_t* __restrict__ bcflag,
+                                T* __restrict__ A) {
+  constexpr int NEN = 1 << DIM, NK = DIM == 3 ? 27 : 9;
+  const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+  if (t >= g.N * NK) return;
+  const int k = (int)(t / g.N);
+  const long long n = t - k * g.N;
+  long long li, lj, lk;
+  lattice3(n, g.nn[0], g.nn[1], g.N, li, lj, lk);
+  const int o[3] = {k % 3 - 1, (k / 3) % 3 - 1, DIM == 3 ? k / 9 - 1 : 0};
+  const int p[3] = {(int)li, (int)lj, (int)lk};
+  double v[DIM][DIM] = {};
+  int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
+  bool in = true;
+#pragma unroll
+  for (int d = 0; d < DIM; d++) {
+    in = in && p[d] + o[d] >= 0 && p[d] + o[d] <= g.res[d];
+    lo[d] = max(max(p[d], p[d] + o[d]) - 1, 0);
+    hi[d] = min(min(p[d], p[d] + o[d]), g.res[d] - 1);
+  }
+  if (in) {
+    for (int ek = lo[2]; ek <= hi[2]; ek++)
+      for (int ej = lo[1]; ej <= hi[1]; ej++)
+        for (int ei = lo[0]; ei <= hi[0]; ei++) {
+          const int a = (p[0] - ei) + 2 * (p[1] - ej) + (DIM == 3 ? 4 * (p[2] - ek) : 0);
+          const int b = a + o[0] + 2 * o[1] + 4 * o[2];
+          for (int d = 0; d < DIM; d++) {
+            double u[NEN][DIM], ye[NEN][DIM];
+#pragma unroll
+            for (int q = 0; q < NEN; q++)
+#pragma unroll
+              for (int c = 0; c < DIM; c++) u[q][c] = q == b && c == d ? 1.0 : 0.0;
+            if constexpr (DIM == 3) {
+              const double ix = 0.25 / (vcoord_t(g, 0, ei + 1) - vcoord_t(g, 0, ei));
+              const double iy = 0.25 / (vcoord_t(g, 1, ej + 1) - vcoord_t(g, 1, ej));
+              const double iz = 0.25 / (vcoord_t(g, 2, ek + 1) - vcoord_t(g, 2, ek));
+              double P[3][4], Q[3][4], R[3][4], M[27], m[30];
+              grad_coeffs3(u, ix, iy, iz, P, Q, R);
+              load_moments3(g, Mom, ei, ej, ek, M);
+              element_moments3(P, Q, R, M, m);
+              epilogue3(m, ix, iy, iz, ye);
+            } else {
+              const double ix = 0.5 / (vcoord_t(g, 0, ei + 1) - vcoord_t(g, 0, ei));
+              const double iy = 0.5 / (vcoord_t(g, 1, ej + 1) - vcoord_t(g, 1, ej));
+              element2(u, ix, iy, 0, Mom, g.E, ei + (long long)g.res[0] * ej, (const double4*)nullptr, 0, 0, ye);
+            }
+#pragma unroll
+            for (int q = 0; q < NEN; q++)
+              if (q == a)
+#pragma unroll
+                for (int c = 0; c < DIM; c++)
+#pragma unroll
+                  for (int d2 = 0; d2 < DIM; d2++)
+                    if (d2 == d) v[c][d2] += ye[q][c];
+          }
+        }
+  }
+  const unsigned bf = bcflag ? bcflag[n] : 0u;
+  const long long nd = g.N * DIM;
+#pragma unroll
+  for (int d = 0; d < DIM; d++)
+#pragma unroll
+    for (int c = 0; c < DIM; c++) A[((long long)k * DIM + d) * nd + n * DIM + c] = ((bf >> c) & 1u) ? (T)0 : (T)v[c][d];
+}
+
+template <typename T>
+void launch_stencil_build(const Geo& g, const double* Mom, const uint8_t* bcflag, T* A, hipStream_t st) {
+  const long long nt = g.N * (g.dim == 3 ? 27 : 9);
+  const dim3 nb((unsigned)((nt + kBlock - 1) / kBlock));
+  if (g.dim == 3)
+    hipLaunchKernelGGL((k_stencil_build<T, 3>), nb, dim3(kBlock), 0, st, g, Mom, bcflag, A);
+  else
+    hipLaunchKernelGGL((k_stencil_build<T, 2>), nb, dim3(kBlock), 0, st, g, Mom, bcflag, A);
+}
+template void launch_stencil_build<double>(const Geo&, const double*, const uint8_t*, double*, hipStream_t);
+template void launch_stencil_build<float>(const Geo&, const double*, const uint8_t*, float*, hipStream_t);
 
 // ---------------------------------------------------------------------------
 // Dense operator of a coarsest level
