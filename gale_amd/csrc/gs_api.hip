@@ -188,6 +188,7 @@ struct gs_solver {
   float *x32 = nullptr, *y32 = nullptr;
   double* S = nullptr;
   double* hS = nullptr;
+  double* hP = nullptr;  // pinned: partial sums of b.b and r.r of the inner CG
   Reducer rd{};
   double* cg_z = nullptr;
   bool for_batch = false;  // hierarchy for the batched kernel: small coarsest level, no direct solve
@@ -248,7 +249,7 @@ extern "C" int32_t gs_device_count(void) {
 }
 
 static int32_t alloc_reducer(Reducer* rd) {
-  CK(dalloc(&rd->partials, (long long)kMaxReduceBlocks * 4));
+  CK(dalloc(&rd->partials, kReducerDoubles));
   return GS_OK;
 }
 
@@ -1177,6 +1178,8 @@ extern "C" int32_t gs_solver_create(gs_problem* pb, const gs_uzawa_params* up, g
     return fail(GS_E_HIP);
   s->P_alloc = P;
   if (hipHostMalloc(reinterpret_cast<void**>(&s->hS), sizeof(double) * S_COUNT) != hipSuccess) return fail(GS_E_HIP);
+  if (hipHostMalloc(reinterpret_cast<void**>(&s->hP), sizeof(double) * 2 * kMaxReduceBlocks) != hipSuccess)
+    return fail(GS_E_HIP);
   if (alloc_reducer(&s->rd)) return fail(GS_E_HIP);
   if (hipEventCreate(&s->e0) != hipSuccess || hipEventCreate(&s->e1) != hipSuccess) return fail(GS_E_HIP);
   hipStream_t st = pb->st;
@@ -1200,6 +1203,7 @@ extern "C" void gs_solver_destroy(gs_solver* s) {
   dfree(s->yielded); dfree(s->x32); dfree(s->y32); dfree(s->S); dfree(s->rd.partials);
   dfree(s->logeta); dfree(s->rec_r0); dfree(s->rec_p0); dfree(s->fl_s); dfree(s->fl_q); dfree(s->fl_aux);
   if (s->hS) (void)hipHostFree(s->hS);
+  if (s->hP) (void)hipHostFree(s->hP);
   if (s->e0) (void)hipEventDestroy(s->e0);
   if (s->e1) (void)hipEventDestroy(s->e1);
   delete s;
@@ -1554,22 +1558,19 @@ static T* vcycle(gs_solver* s, int l, const T* b0 = nullptr, T* out = nullptr) {
   return cheb_smooth<T>(L, nu, x, st, b, out, &beta0);
 }
 
-// z = M^-1 r by one V-cycle (FP64, or FP32 in the mixed-precision mode).
-static void mg_precond(gs_solver* s, const double* r, double* z) {
-  MGLevel& L = s->mg.lv[0];
-  hipStream_t st = s->pb->st;
-  if (s->mg.L == 0 && s->mg.nfc > 0) {
-    // the whole mesh is solved directly, in FP64 also in the mixed mode:
-    // without a smoother an inverse rounded to FP32 stops preconditioning
-    // once the condition number passes 1e7
-    vcycle<double>(s, 0, r, z);
-  } else if (s->up.precision == GS_PREC_MIXED) {
-    launch_d2f(r, L.bf, L.n, st);
-    const float* x = vcycle<float>(s, 0);
-    launch_f2d(x, z, L.n, st);
-  } else {
-    vcycle<double>(s, 0, r, z);
-  }
+// One V-cycle from the inner CG's residual, in FP64 (cg_r to cg_z) or, in the
+// mixed-precision mode, in FP32 (the finest level's b, which the CG writes
+// with its residual, to the buffer returned in *z32).  A mesh that is solved
+// directly is so in FP64 also in the mixed mode: without a smoother an inverse
+// rounded to FP32 stops preconditioning once the condition number passes 1e7.
+static bool mg_fp32(const gs_solver* s) {
+  return s->up.precision == GS_PREC_MIXED && !(s->mg.L == 0 && s->mg.nfc > 0);
+}
+static void mg_precond(gs_solver* s, const float** z32) {
+  if (mg_fp32(s))
+    *z32 = vcycle<float>(s, 0);
+  else
+    vcycle<double>(s, 0, s->cg_r, s->cg_z);
 }
 
 // The fused constitutive pass + diagonal operators + right-hand sides.
@@ -1748,51 +1749,63 @@ static int32_t inner_solve_mg(gs_solver* s, const double* b, double* x, double r
   hipStream_t st = pb->st;
   const long long n = s->n;
   MGLevel& L0 = s->mg.lv[0];
-  launch_fill(x, n, 0.0, st);
-  CK(hipMemcpyAsync(s->cg_r, b, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
   // b.b is read back with the first convergence check, not before the first
   // iteration (one host round trip fewer per inner solve).  With b = 0 every
   // iterate stays exactly zero (the V-cycle of 0 is 0 and alpha, beta are
   // guarded), so that case still returns x = 0 after no counted iteration.
-  launch_dot(b, b, n, s->S, S_BB, s->rd, st);
-  mg_precond(s, s->cg_r, s->cg_z);
-  CK(hipMemcpyAsync(s->cg_p, s->cg_z, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
-  launch_dot(s->cg_r, s->cg_z, n, s->S, S_RZ, s->rd, st);
+  float* rf = mg_fp32(s) ? L0.bf : nullptr;
+  const float* z32 = nullptr;
+  launch_fcg_start(b, x, s->cg_r, rf, n, s->rd, st);
+  mg_precond(s, &z32);
+  if (z32)
+    launch_fcg_first<float>(s->cg_p, z32, s->cg_r, n, s->S, s->rd, st);
+  else
+    launch_fcg_first<double>(s->cg_p, s->cg_z, s->cg_r, n, s->S, s->rd, st);
   const int maxit = s->up.inner_max_iterations;
   // Convergence is checked after every iteration: a V-cycle iteration costs
   // far more than the host round trip, and stopping one iteration earlier
   // pays for many of them (over ten 96^3 fields the learned solve took 5 %
   // less time than with a check every second iteration, faster on all ten;
   // the plain solve the same time).  check_every paces the Jacobi CG.
-  const int every = 1;
+  const int nb = fcg_blocks(n);
   int k = 0;
-  bool conv = false, first = true;
+  bool conv = false;
   double target = 0.0;
   while (k < maxit) {
     launch_mom_apply<double>(L0.g, s->cg_p, s->cg_Ap, L0.M64, pb->bcflag, L0.h64, st);
     s->k_applies++;
-    launch_dot(s->cg_p, s->cg_Ap, n, s->S, S_PAP, s->rd, st);
-    launch_fcg_update(x, s->cg_r, s->cg_p, s->cg_Ap, n, s->S, s->rd, st);
+    launch_fcg_pap(s->cg_p, s->cg_Ap, n, s->rd, st);
+    launch_fcg_update(x, s->cg_r, rf, s->cg_p, s->cg_Ap, n, k, s->S, s->rd, st);
+    // the host adds the blocks' partial sums (in block order)
+    const bool first = k == 0;
     k++;
-    if (k % every == 0 || k >= maxit) {
-      CKS(read_scalars(s));
-      if (first) {
-        first = false;
-        const double bb = s->hS[S_BB];
-        if (bb == 0.0) return GS_OK;
-        if (!std::isfinite(bb)) return GS_E_NAN;
-        target = rtol * rtol * bb;
-      }
-      const double rr = s->hS[S_RR];
-      if (!std::isfinite(rr)) return GS_E_NAN;
-      if (rr <= target) {
-        conv = true;
-        break;
-      }
+    const int from = first ? kPartBB : kPartRR, cnt = first ? kMaxReduceBlocks + nb : nb;
+    CK(hipMemcpyAsync(s->hP, s->rd.partials + from, sizeof(double) * cnt, hipMemcpyDeviceToHost, st));
+    CK(hipStreamSynchronize(st));
+    const double* hrr = s->hP + (first ? kMaxReduceBlocks : 0);
+    if (first) {
+      double bb = 0.0;
+      for (int i = 0; i < nb; i++) bb += s->hP[i];
+      if (bb == 0.0) return GS_OK;
+      if (!std::isfinite(bb)) return GS_E_NAN;
+      target = rtol * rtol * bb;
     }
-    mg_precond(s, s->cg_r, s->cg_z);
-    launch_fcg_dots(s->cg_z, s->cg_r, s->cg_Ap, n, s->S, s->rd, st);
-    launch_fcg_p(s->cg_p, s->cg_z, n, s->S, st);
+    double rr = 0.0;
+    for (int i = 0; i < nb; i++) rr += hrr[i];
+    if (!std::isfinite(rr)) return GS_E_NAN;
+    if (rr <= target) {
+      conv = true;
+      break;
+    }
+    if (k >= maxit) break;
+    mg_precond(s, &z32);
+    if (z32) {
+      launch_fcg_dots<float>(z32, s->cg_r, s->cg_Ap, n, s->rd, st);
+      launch_fcg_p<float>(s->cg_p, z32, n, k - 1, s->S, s->rd, st);
+    } else {
+      launch_fcg_dots<double>(s->cg_z, s->cg_r, s->cg_Ap, n, s->rd, st);
+      launch_fcg_p<double>(s->cg_p, s->cg_z, n, k - 1, s->S, s->rd, st);
+    }
   }
   *its += k;
   if (!conv) return GS_E_INNER_MAXIT;

@@ -36,6 +36,7 @@ enum Slot {
   S_BB = 3,      // b . b (inner)
   S_BETA = 4,    // inner beta
   S_ALPHA = 5,   // inner alpha (flexible CG)
+  S_RZ2 = 6,     // r.z of the flexible CG alternates between S_RZ and S_RZ2
   S_ZR = 8,      // Uzawa z . r
   S_ZR_PREV = 9,
   S_UBETA = 10,  // Uzawa beta
@@ -56,11 +57,18 @@ enum Slot {
 };
 
 struct Reducer {
-  double* partials;   // >= kMaxReduceBlocks * 4 doubles (block partial sums)
+  double* partials;   // kReducerDoubles doubles (block partial sums)
 };
 
 constexpr int kBlock = 256;
 constexpr int kMaxReduceBlocks = 1024;
+// Partial sums: four values a block for the reductions that finish in a launch
+// of their own, then those of the flexible CG, which its next kernel (or the
+// host) adds up: b.b and r.r (side by side, read by the host), p.Ap, and z.r
+// with z.Ap.
+constexpr int kPartBB = 4 * kMaxReduceBlocks, kPartRR = 5 * kMaxReduceBlocks, kPartPAP = 6 * kMaxReduceBlocks,
+              kPartZ = 7 * kMaxReduceBlocks;
+constexpr long long kReducerDoubles = 9LL * kMaxReduceBlocks;
 
 // Fused constitutive pass inputs.
 struct SetupArgs {
@@ -127,12 +135,21 @@ void launch_cg_update(double* x, double* r, const double* p, const double* Ap, c
 void launch_cg_pupdate(double* p, const double* r, const double* dinv, long long n, const double* S,
                        hipStream_t st);
 
-// Flexible (Polak-Ribiere) CG with a variable preconditioner.
-void launch_fcg_update(double* x, double* r, const double* p, const double* Ap, long long n, double* S, Reducer rd,
-                       hipStream_t st);
-void launch_fcg_dots(const double* z, const double* r, const double* Ap, long long n, double* S, Reducer rd,
-                     hipStream_t st);
-void launch_fcg_p(double* p, const double* z, long long n, const double* S, hipStream_t st);
+// Flexible (Polak-Ribiere) CG with a variable preconditioner z = M^-1 r in
+// FP64 or FP32 (rf: FP32 copy of r, or null).  Partial sums go to the
+// reducer's flexible CG slots; it: iteration from 0.
+void launch_fcg_start(const double* b, double* x, double* r, float* rf, long long n, Reducer rd, hipStream_t st);
+template <typename T>
+void launch_fcg_first(double* p, const T* z, const double* r, long long n, double* S, Reducer rd, hipStream_t st);
+void launch_fcg_pap(const double* p, const double* Ap, long long n, Reducer rd, hipStream_t st);
+void launch_fcg_update(double* x, double* r, float* rf, const double* p, const double* Ap, long long n, int it,
+                       double* S, Reducer rd, hipStream_t st);
+template <typename T>
+void launch_fcg_dots(const T* z, const double* r, const double* Ap, long long n, Reducer rd, hipStream_t st);
+template <typename T>
+void launch_fcg_p(double* p, const T* z, long long n, int it, double* S, Reducer rd, hipStream_t st);
+// Blocks (partial sums a value) of the flexible CG reductions over n entries.
+int fcg_blocks(long long n);
 
 // Uzawa outer loop.
 void launch_uz_precond(const double* r, const double* Qinv, double* z, long long n, double* S, Reducer rd,

@@ -270,69 +270,122 @@ void launch_cg_pupdate(double* p, const double* r, const double* dinv, long long
   hipLaunchKernelGGL(k_cg_pupdate, dim3(grid_for(n)), dim3(kBlock), 0, st, p, r, dinv, n, S);
 }
 
-// Flexible CG: alpha = rz / pAp; x += alpha p; r -= alpha Ap.
-__global__ void k_fcg_update(double* __restrict__ x, double* __restrict__ r, const double* __restrict__ p,
-                             const double* __restrict__ Ap, long long n, double* S, Reducer rd) {
-  const double rz = S[S_RZ], pap = S[S_PAP];
-  const double alpha = (pap != 0.0 && isfinite(pap)) ? rz / pap : 0.0;
+// Flexible CG.  Each kernel that needs the sums of the one before adds its
+// blocks' partial sums itself (sum_partials), and the host adds those of r.r:
+// a one-block launch to finish a reduction cost 2-4 us and a gap, three times
+// an iteration.  r.z alternates between two slots so that no block reads the
+// one that block 0 writes.
+int fcg_blocks(long long n) { return reduce_grid(n); }
+
+__device__ __forceinline__ int fcg_rz_slot(int it) { return (it & 1) ? S_RZ2 : S_RZ; }
+
+__global__ void k_fcg_start(const double* __restrict__ b, double* __restrict__ x, double* __restrict__ r,
+                            float* __restrict__ rf, long long n, Reducer rd) {
+  double v[1] = {0.0};
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
+    const double bi = b[i];
+    x[i] = 0.0;
+    r[i] = bi;
+    if (rf) rf[i] = (float)bi;
+    v[0] += bi * bi;
+  }
+  block_partials<1, false>(v, rd);
+}
+void launch_fcg_start(const double* b, double* x, double* r, float* rf, long long n, Reducer rd, hipStream_t st) {
+  rd.partials += kPartBB;
+  hipLaunchKernelGGL(k_fcg_start, dim3(fcg_blocks(n)), dim3(kBlock), 0, st, b, x, r, rf, n, rd);
+}
+
+template <typename T>
+__global__ void k_fcg_first(double* __restrict__ p, const T* __restrict__ z, const double* __restrict__ r, long long n,
+                            Reducer rd) {
+  double v[1] = {0.0};
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
+    const double zi = (double)z[i];
+    p[i] = zi;
+    v[0] += zi * r[i];
+  }
+  block_partials<1, false>(v, rd);
+}
+template <typename T>
+void launch_fcg_first(double* p, const T* z, const double* r, long long n, double* S, Reducer rd, hipStream_t st) {
+  const int nb = fcg_blocks(n);
+  hipLaunchKernelGGL(k_fcg_first<T>, dim3(nb), dim3(kBlock), 0, st, p, z, r, n, rd);
+  reduce_finish<1, false>(rd, nb, OpStore{S, S_RZ}, st);
+}
+template void launch_fcg_first<double>(double*, const double*, const double*, long long, double*, Reducer, hipStream_t);
+template void launch_fcg_first<float>(double*, const float*, const double*, long long, double*, Reducer, hipStream_t);
+
+void launch_fcg_pap(const double* p, const double* Ap, long long n, Reducer rd, hipStream_t st) {
+  rd.partials += kPartPAP;
+  hipLaunchKernelGGL(k_dot, dim3(fcg_blocks(n)), dim3(kBlock), 0, st, p, Ap, n, nullptr, 0, rd);
+}
+
+// alpha = rz / pAp; x += alpha p; r -= alpha Ap.
+__global__ void k_fcg_update(double* __restrict__ x, double* __restrict__ r, float* __restrict__ rf,
+                             const double* __restrict__ p, const double* __restrict__ Ap, long long n, int it,
+                             double* S, const double* __restrict__ pap_part, Reducer rd) {
+  double pap[1];
+  sum_partials<1>(pap_part, gridDim.x, pap);
+  const double rz = S[fcg_rz_slot(it)];
+  const double alpha = (pap[0] != 0.0 && isfinite(pap[0])) ? rz / pap[0] : 0.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) S[S_ALPHA] = alpha;
   double v[1] = {0.0};
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
     x[i] += alpha * p[i];
     const double ri = r[i] - alpha * Ap[i];
     r[i] = ri;
+    if (rf) rf[i] = (float)ri;
     v[0] += ri * ri;
   }
   block_partials<1, false>(v, rd);
 }
-struct OpFcgUpdate {
-  double* S;
-  __device__ void operator()(const double* t) const {
-    const double rz = S[S_RZ], pap = S[S_PAP];
-    S[S_RR] = t[0];
-    S[S_ALPHA] = (pap != 0.0 && isfinite(pap)) ? rz / pap : 0.0;
-  }
-};
-void launch_fcg_update(double* x, double* r, const double* p, const double* Ap, long long n, double* S, Reducer rd,
-                       hipStream_t st) {
-  const int nb = reduce_grid(n);
-  hipLaunchKernelGGL(k_fcg_update, dim3(nb), dim3(kBlock), 0, st, x, r, p, Ap, n, S, rd);
-  reduce_finish<1, false>(rd, nb, OpFcgUpdate{S}, st);
+void launch_fcg_update(double* x, double* r, float* rf, const double* p, const double* Ap, long long n, int it,
+                       double* S, Reducer rd, hipStream_t st) {
+  const double* pap = rd.partials + kPartPAP;
+  rd.partials += kPartRR;
+  hipLaunchKernelGGL(k_fcg_update, dim3(fcg_blocks(n)), dim3(kBlock), 0, st, x, r, rf, p, Ap, n, it, S, pap, rd);
 }
 
 // z.r and z.Ap; beta = (z.(r_new - r_old)) / rz_old = -alpha z.Ap / rz_old (Polak-Ribiere).
-__global__ void k_fcg_dots(const double* __restrict__ z, const double* __restrict__ r, const double* __restrict__ Ap,
-                           long long n, double* S, Reducer rd) {
+template <typename T>
+__global__ void k_fcg_dots(const T* __restrict__ z, const double* __restrict__ r, const double* __restrict__ Ap,
+                           long long n, Reducer rd) {
   double v[2] = {0.0, 0.0};
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    const double zi = z[i];
+    const double zi = (double)z[i];
     v[0] += zi * r[i];
     v[1] += zi * Ap[i];
   }
   block_partials<2, false>(v, rd);
 }
-struct OpFcgDots {
-  double* S;
-  __device__ void operator()(const double* t) const {
-    const double rz = S[S_RZ];
-    S[S_BETA] = rz != 0.0 ? -S[S_ALPHA] * t[1] / rz : 0.0;
-    S[S_RZ] = t[0];
-  }
-};
-void launch_fcg_dots(const double* z, const double* r, const double* Ap, long long n, double* S, Reducer rd,
-                     hipStream_t st) {
-  const int nb = reduce_grid(n);
-  hipLaunchKernelGGL(k_fcg_dots, dim3(nb), dim3(kBlock), 0, st, z, r, Ap, n, S, rd);
-  reduce_finish<2, false>(rd, nb, OpFcgDots{S}, st);
+template <typename T>
+void launch_fcg_dots(const T* z, const double* r, const double* Ap, long long n, Reducer rd, hipStream_t st) {
+  rd.partials += kPartZ;
+  hipLaunchKernelGGL(k_fcg_dots<T>, dim3(fcg_blocks(n)), dim3(kBlock), 0, st, z, r, Ap, n, rd);
 }
+template void launch_fcg_dots<double>(const double*, const double*, const double*, long long, Reducer, hipStream_t);
+template void launch_fcg_dots<float>(const float*, const double*, const double*, long long, Reducer, hipStream_t);
 
-__global__ void k_fcg_p(double* __restrict__ p, const double* __restrict__ z, long long n, const double* S) {
-  const double beta = S[S_BETA];
+// p = z + beta p after iteration it; r.z of the next one.
+template <typename T>
+__global__ void k_fcg_p(double* __restrict__ p, const T* __restrict__ z, long long n, int it, double* S,
+                        const double* __restrict__ z_part, int nb) {
+  double t[2];
+  sum_partials<2>(z_part, nb, t);
+  const double rz = S[fcg_rz_slot(it)];
+  const double beta = rz != 0.0 ? -S[S_ALPHA] * t[1] / rz : 0.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) S[fcg_rz_slot(it + 1)] = t[0];
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-    p[i] = z[i] + beta * p[i];
+    p[i] = (double)z[i] + beta * p[i];
 }
-void launch_fcg_p(double* p, const double* z, long long n, const double* S, hipStream_t st) {
-  hipLaunchKernelGGL(k_fcg_p, dim3(grid_for(n)), dim3(kBlock), 0, st, p, z, n, S);
+template <typename T>
+void launch_fcg_p(double* p, const T* z, long long n, int it, double* S, Reducer rd, hipStream_t st) {
+  const int nb = fcg_blocks(n);
+  hipLaunchKernelGGL(k_fcg_p<T>, dim3(nb), dim3(kBlock), 0, st, p, z, n, it, S, rd.partials + kPartZ, nb);
 }
+template void launch_fcg_p<double>(double*, const double*, long long, int, double*, Reducer, hipStream_t);
+template void launch_fcg_p<float>(double*, const float*, long long, int, double*, Reducer, hipStream_t);
 
 // ---------------------------------------------------------------------------
 // Uzawa outer loop vector steps (Stokes_SLE_UzawaSolver.cxx:664-837).

@@ -11,7 +11,6 @@ void launch_moments_coarsen(const Geo& gc, const Geo& gf, const double* Mf, doub
 void launch_d2f(const double* a, float* b, long long n, hipStream_t st);
 // FP32 copy of a level's moments, layout-aware (gs_tile.h mom_index).
 void launch_mom_d2f(const Geo& g, const double* a, float* b, hipStream_t st);
-void launch_f2d(const float* a, double* b, long long n, hipStream_t st);
 // Moment-form K apply (tiled, gs_tile.hip); Mom in the layout of gs_tile.h
 // (mom_index: tile-major in 3D, SoA in 2D); halo
 // needs tile_halo_size(g) values.
@@ -29,8 +28,6 @@ void launch_cheb(const T* b, const T* Ax, const T* dinv, T* d, T* x, long long n
 // assembled level, one launch.
 template <typename T>
 void launch_stencil_epi(const Geo& g, const T* A, const T* x, const TileEpi<T>& ep, hipStream_t st);
-template <typename T>
-void launch_resid(const T* b, const T* Ax, T* r, long long n, hipStream_t st);
 // Dense coarsest solve x = Kinv b on the free dofs (nf at most
 // kDenseWideMax, rows of ld values), zero on the others (pos < 0).
 constexpr int kDenseWideMax = 8192;

@@ -170,9 +170,6 @@ void launch_mom_d2f(const Geo& g, const double* a, float* b, hipStream_t st) {
 void launch_d2f(const double* a, float* b, long long n, hipStream_t st) {
   if (n > 0) hipLaunchKernelGGL((k_convert<double, float>), dim3(gridn(n) < 8192 ? gridn(n) : 8192), dim3(kBlock), 0, st, a, b, n);
 }
-void launch_f2d(const float* a, double* b, long long n, hipStream_t st) {
-  if (n > 0) hipLaunchKernelGGL((k_convert<float, double>), dim3(gridn(n) < 8192 ? gridn(n) : 8192), dim3(kBlock), 0, st, a, b, n);
-}
 
 template <typename T>
 __global__ void k_fill_mg(T* __restrict__ y, long long n, T v) {
@@ -507,21 +504,6 @@ void launch_stencil_epi(const Geo& g, const T* A, const T* x, const TileEpi<T>& 
 }
 template void launch_stencil_epi<double>(const Geo&, const double*, const double*, const TileEpi<double>&, hipStream_t);
 template void launch_stencil_epi<float>(const Geo&, const float*, const float*, const TileEpi<float>&, hipStream_t);
-
-// r = b - Ax
-template <typename T>
-__global__ void k_resid(const T* __restrict__ b, const T* __restrict__ Ax, T* __restrict__ r, long long n) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-    r[i] = b[i] - Ax[i];
-}
-template <typename T>
-void launch_resid(const T* b, const T* Ax, T* r, long long n, hipStream_t st) {
-  unsigned gb = gridn(n);
-  if (gb > 8192) gb = 8192;
-  hipLaunchKernelGGL(k_resid<T>, dim3(gb), dim3(kBlock), 0, st, b, Ax, r, n);
-}
-template void launch_resid<double>(const double*, const double*, double*, long long, hipStream_t);
-template void launch_resid<float>(const float*, const float*, float*, long long, hipStream_t);
 
 // Dense coarse solve: x[free[i]] = sum_j Kinv[i][j] b[free[j]], zero on the
 // Dirichlet dofs.  16 rows per 1024-thread workgroup, one wavefront per row;
