@@ -98,6 +98,8 @@ struct gs_problem {
   double* hS = nullptr;  // pinned
   Reducer rd{};
   bool min_one_particle = true;
+  double* out_xw = nullptr;  // local coordinates and weights in caller order (particle read-back)
+  long long out_n = 0;       // particles it holds
   double* halo64 = nullptr;  // tiled K apply scratch (fine level)
   float* halo32 = nullptr;
   int wkind = GS_WEIGHTS_CONSTANT;  // integration weights of the material points
@@ -303,25 +305,20 @@ static int32_t relocate(gs_problem* pb) {
   launch_offsets(reinterpret_cast<const int*>(pb->keys), P, pb->g.E, pb->off, st);
   launch_remap(pb->g, pb->coord, pb->keys, pb->pk, P, st);
   pb->pk32_valid = false;
+  launch_cell_counts(pb->off, pb->g.E, pb->S, st);
   CK(hipMemcpyAsync(pb->hS, pb->S, sizeof(double) * S_COUNT, hipMemcpyDeviceToHost, st));
   CK(hipStreamSynchronize(st));
   unsigned esc;
   std::memcpy(&esc, pb->hS + S_ESC, sizeof(unsigned));
   pb->escaped = esc;
+  int cells[2];
+  std::memcpy(cells, pb->hS + S_CELLS, sizeof(cells));
   // every element must hold at least one material point (ConstantWeights divides by the count)
-  std::vector<int> off(pb->g.E + 1);
-  CK(hipMemcpy(off.data(), pb->off, sizeof(int) * (pb->g.E + 1), hipMemcpyDeviceToHost));
-  pb->min_one_particle = true;
-  for (long long e = 0; e < pb->g.E; e++)
-    if (off[e + 1] == off[e]) {
-      pb->min_one_particle = false;
-      break;
-    }
+  pb->min_one_particle = cells[1] == 0;
   if (pb->wkind == GS_WEIGHTS_DVC && P > 0) {
     // DVCWeights: integration point at the centroid of its discrete Voronoi
     // region, weight = the region's volume (gs_weights.hip)
-    int maxp = 0;
-    for (long long e = 0; e < pb->g.E; e++) maxp = std::max(maxp, off[e + 1] - off[e]);
+    const int maxp = cells[0];
     if (maxp > dvc_max_particles(pb->dim, pb->wres)) return GS_E_INVALID;
     const int32_t r = dvc_weights(pb->dim, pb->wres, pb->g.E, pb->off, pb->pid, pb->pk, pb->wp, maxp, st);
     if (r != GS_OK) return r;
@@ -477,7 +474,7 @@ extern "C" void gs_problem_destroy(gs_problem* pb) {
   dfree(pb->eta0p); dfree(pb->eta0p2); dfree(pb->off); dfree(pb->keys); dfree(pb->keys2); dfree(pb->vals);
   dfree(pb->wp); dfree(pb->pstr); dfree(pb->pstr2); dfree(pb->pinc); dfree(pb->pinc2);
   dfree(pb->vals2); dfree(pb->S); dfree(pb->rd.partials); dfree(pb->halo64);
-  dfree(pb->halo32);
+  dfree(pb->halo32); dfree(pb->out_xw);
   if (pb->sort_tmp) (void)hipFree(pb->sort_tmp);
   if (pb->hS) (void)hipHostFree(pb->hS);
   if (pb->st) (void)hipStreamDestroy(pb->st);
@@ -498,46 +495,29 @@ extern "C" int32_t gs_problem_particles(gs_problem* pb, double* coord, int32_t* 
   if (!pb) return GS_E_INVALID;
   const long long P = pb->P, E = pb->g.E;
   const int dim = pb->dim;
-  CK(hipStreamSynchronize(pb->st));
-  std::vector<int> pid(P > 0 ? P : 1);
-  std::vector<unsigned> keys(P > 0 ? P : 1);
-  CK(hipMemcpy(pid.data(), pb->pid, sizeof(int) * P, hipMemcpyDeviceToHost));
-  CK(hipMemcpy(keys.data(), pb->keys, sizeof(unsigned) * P, hipMemcpyDeviceToHost));
-  if (coord) {
-    std::vector<double> c(3 * P > 0 ? 3 * P : 1);
-    CK(hipMemcpy(c.data(), pb->coord, sizeof(double) * 3 * P, hipMemcpyDeviceToHost));
-    for (long long i = 0; i < P; i++)
-      for (int d = 0; d < 3; d++) coord[3 * (long long)pid[i] + d] = c[3 * i + d];
+  hipStream_t st = pb->st;
+  CK(hipStreamSynchronize(st));
+  if (P == 0 || !(coord || owner || xi || weight)) return GS_OK;
+  // the device puts the state in caller order (coordinates and owners through
+  // the buffers the next relocation sorts into), so each output is one copy
+  // straight into the caller's array
+  if ((xi || weight) && pb->out_n != P) {
+    dfree(pb->out_xw);
+    pb->out_n = 0;
+    CK(dalloc(&pb->out_xw, (dim + 1) * P));
+    pb->out_n = P;
   }
-  if (owner)
-    for (long long i = 0; i < P; i++) owner[pid[i]] = keys[i] >= (unsigned)E ? -1 : (int32_t)keys[i];
-  if (xi || weight) {
-    std::vector<double4> pk(P > 0 ? P : 1);
-    std::vector<int> off(E + 1);
-    CK(hipMemcpy(pk.data(), pb->pk, sizeof(double4) * P, hipMemcpyDeviceToHost));
-    CK(hipMemcpy(off.data(), pb->off, sizeof(int) * (E + 1), hipMemcpyDeviceToHost));
-    std::vector<double> wv;
-    if (pb->wkind == GS_WEIGHTS_DVC && P > 0) {
-      wv.resize(P);
-      CK(hipMemcpy(wv.data(), pb->wp, sizeof(double) * P, hipMemcpyDeviceToHost));
-    }
-    for (long long e = 0; e < E; e++)
-      for (int i = off[e]; i < off[e + 1]; i++) {
-        const long long o = pid[i];
-        if (xi) {
-          xi[o * dim] = pk[i].x;
-          xi[o * dim + 1] = pk[i].y;
-          if (dim == 3) xi[o * dim + 2] = pk[i].z;
-        }
-        if (weight) weight[o] = wv.empty() ? (dim == 2 ? 4.0 : 8.0) / (double)(off[e + 1] - off[e]) : wv[i];
-      }
-    for (long long i = off[E]; i < P; i++) {
-      const long long o = pid[i];
-      if (xi)
-        for (int d = 0; d < dim; d++) xi[o * dim + d] = 0.0;
-      if (weight) weight[o] = 0.0;
-    }
-  }
+  double* xi_d = xi ? pb->out_xw : nullptr;
+  double* w_d = weight ? pb->out_xw + (long long)dim * P : nullptr;
+  launch_particles_out(dim, P, E, pb->pid, pb->keys, pb->off, pb->coord, pb->pk,
+                       pb->wkind == GS_WEIGHTS_DVC ? pb->wp : nullptr, coord ? pb->coord2 : nullptr,
+                       owner ? pb->vals2 : nullptr, xi_d, w_d, st);
+  CK(hipGetLastError());
+  CK(hipStreamSynchronize(st));
+  if (coord) CK(hipMemcpy(coord, pb->coord2, sizeof(double) * 3 * P, hipMemcpyDeviceToHost));
+  if (owner) CK(hipMemcpy(owner, pb->vals2, sizeof(int) * P, hipMemcpyDeviceToHost));
+  if (xi) CK(hipMemcpy(xi, xi_d, sizeof(double) * dim * P, hipMemcpyDeviceToHost));
+  if (weight) CK(hipMemcpy(weight, w_d, sizeof(double) * P, hipMemcpyDeviceToHost));
   return GS_OK;
 }
 
@@ -1089,24 +1069,17 @@ extern "C" int32_t gs_problem_population_control(gs_problem* pb, const gs_pcdvc_
 extern "C" int32_t gs_problem_set_coords(gs_problem* pb, const double* coord) {
   if (!pb || (!coord && pb->P > 0)) return GS_E_INVALID;
   const long long P = pb->P;
-  CK(hipStreamSynchronize(pb->st));
-  std::vector<int> ids(P > 0 ? P : 1);
-  for (long long i = 0; i < P; i++) ids[i] = (int)i;
-  // restore caller order for material / eta0 first
-  std::vector<int> pid(P > 0 ? P : 1), mat(P > 0 ? P : 1), mat_o(P > 0 ? P : 1);
-  CK(hipMemcpy(pid.data(), pb->pid, sizeof(int) * P, hipMemcpyDeviceToHost));
-  CK(hipMemcpy(mat.data(), pb->mat, sizeof(int) * P, hipMemcpyDeviceToHost));
-  for (long long i = 0; i < P; i++) mat_o[pid[i]] = mat[i];
-  for (double* arr : {pb->eta0p, pb->pstr, pb->pinc}) {
-    if (!arr) continue;
-    std::vector<double> e0(P), e0o(P);
-    CK(hipMemcpy(e0.data(), arr, sizeof(double) * P, hipMemcpyDeviceToHost));
-    for (long long i = 0; i < P; i++) e0o[pid[i]] = e0[i];
-    CK(hipMemcpy(arr, e0o.data(), sizeof(double) * P, hipMemcpyHostToDevice));
-  }
-  CK(hipMemcpy(pb->mat, mat_o.data(), sizeof(int) * P, hipMemcpyHostToDevice));
-  CK(hipMemcpy(pb->pid, ids.data(), sizeof(int) * P, hipMemcpyHostToDevice));
-  CK(hipMemcpy(pb->coord, coord, sizeof(double) * 3 * P, hipMemcpyHostToDevice));
+  hipStream_t st = pb->st;
+  // material and the other carried arrays back in caller order first
+  launch_restore_order(P, pb->pid, pb->mat, pb->mat2, PartDoubles{{pb->eta0p, pb->pstr, pb->pinc}},
+                       PartDoubles{{pb->eta0p2, pb->pstr2, pb->pinc2}}, st);
+  CK(hipGetLastError());
+  std::swap(pb->mat, pb->mat2);
+  std::swap(pb->eta0p, pb->eta0p2);
+  std::swap(pb->pstr, pb->pstr2);
+  std::swap(pb->pinc, pb->pinc2);
+  CK(hipStreamSynchronize(st));
+  if (P > 0) CK(hipMemcpy(pb->coord, coord, sizeof(double) * 3 * P, hipMemcpyHostToDevice));
   return relocate(pb);
 }
 

@@ -48,6 +48,7 @@ enum Slot {
   S_TMP2 = 18,
   S_VMAX = 20,
   S_ESC = 24,    // escaped particle count (stored as double)
+  S_CELLS = 25,  // largest particle count of a cell, an empty cell (two ints)
   S_LP_TT = 26,  // learned preconditioner: sum (Q^-1 r)^2
   S_LP_ZQ = 27,  // learned preconditioner: z . q_prev
   S_DS_TT = 28,  // training-pair recording: sum (Q^-1 r)^2, sum e, sum e^2
@@ -172,6 +173,18 @@ void launch_remap(const Geo& g, const double* coord, const unsigned* owner, doub
 void launch_advect_rk2(const Geo& g, double* coord, long long P, const double* u, double dt, double* S,
                        hipStream_t st);
 void launch_vmax(const double* u, long long nnode, int dim, double* S, int slot, Reducer rd, hipStream_t st);
+
+// Particle state in caller order (device buffers, any may be null).
+void launch_particles_out(int dim, long long P, long long E, const int* pid, const unsigned* keys, const int* off,
+                          const double* coord, const double4* pk, const double* wp, double* coord_o, int* owner_o,
+                          double* xi_o, double* w_o, hipStream_t st);
+// Per-particle doubles that move with the particles.
+constexpr int kPartDoubles = 3;
+struct PartDoubles {
+  double* a[kPartDoubles];
+};
+void launch_restore_order(long long P, int* pid, const int* m, int* m2, PartDoubles x, PartDoubles x2, hipStream_t st);
+void launch_cell_counts(const int* off, long long E, double* S, hipStream_t st);
 
 // Element iteration helpers shared by kernels and host.
 inline long long colour_count(const Geo& g, int c) {

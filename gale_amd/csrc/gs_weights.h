@@ -16,13 +16,6 @@ int dvc_weights(int dim, const int* res, long long ncell, const int* off, const 
 // Largest per-cell particle count whose LDS fits kDvcMaxLds.
 long long dvc_max_particles(int dim, const int* res);
 
-// Optional per-particle double arrays that follow the particles (per-particle
-// eta0, StrainWeakening plastic strain and its rate); null entries are skipped.
-constexpr int kPartDoubles = 3;
-struct PartDoubles {
-  double* a[kPartDoubles];
-};
-
 // The sub-grid of one cell's discrete Voronoi diagram.
 struct DvcGrid {
   int dim;
