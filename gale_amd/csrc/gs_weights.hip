@@ -10,7 +10,11 @@
 // within one particle's step every boundary sub-cell is decided on its own,
 // so the 64 lanes decide a step's sub-cells in parallel: the boundary of each
 // particle is a bit set over the sub-cells, the owner of every sub-cell an
-// LDS array.  The result is the reference's, sub-cell for sub-cell.
+// LDS array.  The result is the reference's, sub-cell for sub-cell.  A cell is
+// a chain of short dependent steps, so it is bound by the latency of one: on
+// grids of up to kDvcLaneCells sub-cells (2D's 10 x 10) a lane looks at the
+// sub-cells lane, lane + 64, ..., on larger ones (3D's 10^3) a lane walks the
+// set bits of a boundary word.
 #include <hip/hip_runtime.h>
 
 #include <vector>
@@ -24,6 +28,7 @@ namespace gs {
 namespace {
 
 constexpr int kDvcLanes = 64;
+constexpr int kDvcLaneCells = 256;
 
 // Vertex coordinate of a regular mesh (CartesianGenerator): lo + (i / n)(hi - lo),
 // the end vertices exactly lo and hi.
@@ -152,27 +157,86 @@ __device__ void dvc_grow(const DvcGrid& G, const DvcLds& L, int n) {
   for (int c = lane; c < G.nc; c += kDvcLanes) L.owner[c] = -1;
   for (int q = lane; q < n * G.nwords; q += kDvcLanes) L.bound[q] = 0;
   __syncthreads();
-  // seeds, in order (a later particle in the same sub-cell takes it over)
-  if (lane == 0) {
-    for (int i = 0; i < n; i++) {
+  // Seeds: of several particles in one sub-cell the last owns it.  A particle
+  // owns nothing but its seed then, so its boundary is all the neighbours.
+  for (int i0 = 0; i0 < n; i0 += kDvcLanes) {
+    const int i = i0 + lane;
+    int c = 0;
+    if (i < n) {
       int idx[3] = {0, 0, 0};
       for (int d = 0; d < G.dim; d++) {
         int k = (int)((L.xs[3 * i + d] - (-1.0)) / G.h[d]);
         if (k == G.r[d]) k--;
         idx[d] = k;
       }
-      const int c = idx[0] + G.r[0] * (idx[1] + G.r[1] * idx[2]);
-      L.owner[c] = (short)i;
-      L.bsize[i] = dvc_rebound(G, L.owner, L.cxyz, L.bound + (size_t)i * G.nwords, i, c);
+      c = idx[0] + G.r[0] * (idx[1] + G.r[1] * idx[2]);
+      L.bsize[i] = dvc_rebound(G, L.owner, L.cxyz, L.bound + (size_t)i * G.nwords, -2, c);
+    }
+    // every pass at least one more of the lanes that want a sub-cell is settled
+    for (;;) {
+      const bool want = i < n && L.owner[c] < i;
+      if (!__any(want)) break;
+      if (want) L.owner[c] = (short)i;
+      __syncthreads();
     }
   }
   __syncthreads();
   const double* cx = L.ctr;
   const double* cy = L.ctr + G.r[0];
   const double* cz = L.ctr + G.r[0] + G.r[1];
-  // Rounds of claims until one claims nothing.  Lanes take the boundary's
-  // 32-bit words; a particle with an empty boundary (it claimed nothing last
-  // time) is skipped, as ClaimCells over an empty list claims nothing.
+  // Rounds of claims until one claims nothing; a particle with an empty
+  // boundary (it claimed nothing last time) is skipped, as ClaimCells over an
+  // empty list claims nothing.
+  if (G.nc <= kDvcLaneCells) {
+    constexpr int KC = kDvcLaneCells / kDvcLanes;
+    for (;;) {
+      bool any = false;
+      for (int i = 0; i < n; i++) {
+        if (L.bsize[i] == 0) continue;  // uniform across the wave (LDS value)
+        unsigned* bi = L.bound + (size_t)i * G.nwords;
+        const double* xi_ = L.xs + 3 * i;
+        unsigned mine = 0;  // bit k: sub-cell lane + 64 k is on the boundary
+#pragma unroll
+        for (int k = 0; k < KC; k++) {
+          const int c = lane + kDvcLanes * k;
+          if (c < G.nc) mine |= ((bi[c >> 5] >> (c & 31)) & 1u) << k;
+        }
+        __syncthreads();
+        if (lane < G.nwords) bi[lane] = 0u;
+        unsigned tk = 0;
+#pragma unroll
+        for (int k = 0; k < KC; k++) {
+          if (!((mine >> k) & 1u)) continue;
+          const int c = lane + kDvcLanes * k;
+          const int o = L.owner[c];
+          bool take = o < 0;
+          if (!take && o != i) {
+            const unsigned v = L.cxyz[c];
+            const double c3[3] = {cx[dvc_ix(v)], cy[dvc_iy(v)], G.dim == 3 ? cz[dvc_iz(v)] : 0.0};
+            take = dvc_contest(G.dim, c3, L.xs + 3 * o, xi_) > 0.0;
+          }
+          if (take) {
+            L.owner[c] = (short)i;
+            tk |= 1u << k;
+          }
+        }
+        __syncthreads();
+        int added = 0;
+        if (__any(tk != 0)) {
+          any = true;
+#pragma unroll
+          for (int k = 0; k < KC; k++)
+            if ((tk >> k) & 1u) added += dvc_rebound(G, L.owner, L.cxyz, bi, i, lane + kDvcLanes * k);
+        }
+        const int left = __any(added != 0) ? 1 : 0;  // only whether it is empty matters
+        if (lane == 0) L.bsize[i] = left;
+        __syncthreads();
+      }
+      if (!any) break;
+    }
+    return;
+  }
+  // Lanes take the boundary's 32-bit words.
   for (;;) {
     int total = 0;
     for (int i = 0; i < n; i++) {
