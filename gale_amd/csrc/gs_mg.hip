@@ -4,13 +4,13 @@
 // functions are exactly representable on the fine mesh, the Galerkin coarse
 // operator P^T K P equals the coarse Q1 operator integrated with the SAME
 // material points and weights omega_p = w_p detJ eta_p.  Its element matrix
-// depends on the points only through 27 (3D) / 9 (2D) weighted moments
+// depends on the points only through 27 (3D, 23 of them needed) / 9 (2D) weighted moments
 // M[a,b,c] = sum_p omega_p r^a s^b t^c (a,b,c <= 2) in element-local
 // coordinates, since every entry of B^T D B is a polynomial of degree <= 2 in
 // each local coordinate.  The fine moments come from one pass over the
 // particles; each coarser level's moments are an exact polynomial change of
 // variables of its children's.  Every level is applied matrix-free from its
-// moments (216 B per 3D element instead of 32 B per particle), smoothed by
+// moments (184 B per 3D element instead of 32 B per particle), smoothed by
 // Chebyshev-Jacobi, and the coarsest level is solved with a dense inverse.
 #include "gs_internal.h"
 #include "gs_mg.h"
@@ -80,7 +80,8 @@ __global__ void k_moments_fine(Geo g, const double4* __restrict__ pk, const int*
     }
   }
 #pragma unroll
-  for (int k = 0; k < NM; k++) M[mom_index<double>(g, k, e)] = m[k];
+  for (int k = 0; k < NM; k++)
+    if (DIM == 2 || mom_slot(k) >= 0) M[mom_index<double>(g, k, e)] = m[k];
 }
 
 // Parent moments from children: child local r_f maps to parent r_c = (r_f + sg)/2,
@@ -106,7 +107,7 @@ __global__ void k_moments_coarsen(Geo gc, Geo gf, const double* __restrict__ Mf,
       T[d][2][0] = 0.25; T[d][2][1] = 0.5 * s; T[d][2][2] = 0.25;  // (r+s)^2/4 = (r^2 + 2 s r + 1)/4
     }
     double m[NM];
-    for (int k = 0; k < NM; k++) m[k] = Mf[mom_index<double>(gf, k, e)];
+    for (int k = 0; k < NM; k++) m[k] = DIM == 2 || mom_slot(k) >= 0 ? Mf[mom_index<double>(gf, k, e)] : 0.0;
     if (DIM == 2) {
       for (int b = 0; b < 3; b++)
         for (int a = 0; a < 3; a++) {
@@ -129,7 +130,8 @@ __global__ void k_moments_coarsen(Geo gc, Geo gf, const double* __restrict__ Mf,
     }
   }
 #pragma unroll
-  for (int k = 0; k < NM; k++) Mc[mom_index<double>(gc, k, E)] = acc[k];
+  for (int k = 0; k < NM; k++)
+    if (DIM == 2 || mom_slot(k) >= 0) Mc[mom_index<double>(gc, k, E)] = acc[k];
 }
 
 void launch_moments_fine(const Geo& g, const double4* pk, const int* off, double* M, hipStream_t st) {
@@ -158,7 +160,8 @@ __global__ void k_mom_d2f(Geo g, const double* __restrict__ a, float* __restrict
   const long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x;
   if (e >= g.E) return;
 #pragma unroll
-  for (int k = 0; k < NM; k++) b[mom_index<float>(g, k, e)] = (float)a[mom_index<double>(g, k, e)];
+  for (int k = 0; k < NM; k++)
+    if (DIM == 2 || mom_slot(k) >= 0) b[mom_index<float>(g, k, e)] = (float)a[mom_index<double>(g, k, e)];
 }
 void launch_mom_d2f(const Geo& g, const double* a, float* b, hipStream_t st) {
   if (g.dim == 3)
@@ -202,7 +205,7 @@ __global__ void k_mom_diag(Geo g, int c, long long mcount, const double* __restr
   for (int d = 0; d < DIM; d++) inv[d] = 2.0 / (vcoord_mg(g, d, ijk[d] + 1) - vcoord_mg(g, d, ijk[d]));
   const double cN = DIM == 2 ? 0.25 : 0.125;
   double M[NM];
-  for (int k = 0; k < NM; k++) M[k] = Mom[mom_index<double>(g, k, e)];
+  for (int k = 0; k < NM; k++) M[k] = DIM == 2 || mom_slot(k) >= 0 ? Mom[mom_index<double>(g, k, e)] : 0.0;
   const long long sy = g.nn[0], sz = g.nn[0] * g.nn[1];
   const long long n0 = ijk[0] + sy * ijk[1] + sz * ijk[2];
   for (int a = 0; a < NEN; a++) {

@@ -207,7 +207,7 @@ __device__ __forceinline__ void element_particles3(const T (&A)[3][4], const T (
   }
 }
 
-// The 27 moments of the element at place `local` of apply tile `tile`
+// The moments of the element at place `local` of apply tile `tile`
 // (tile-major layout, gs_tile.h): one 16-byte load per group of
 // G = 16 / sizeof(T) moments, consecutive threads reading consecutive
 // 16-byte slots.  NT marks the loads non-temporal: a stream larger than the
@@ -221,37 +221,41 @@ __device__ __forceinline__ V ld_mom(const V* p) {
   if (NT) return __builtin_nontemporal_load(p);
   return *p;
 }
+// Moment of slot s.
+__device__ constexpr int mom_of_slot(int s) { return s < 17 ? s : (s < 22 ? s + 1 : 24); }
 template <bool NT>
 __device__ __forceinline__ void load_tile_moments3(const double* __restrict__ Mom, long long tile, int local,
                                                    double (&M)[27]) {
-  const double* base = Mom + tile * 27 * kTileThreads;
+  const double* base = Mom + tile * kMom3 * kTileThreads;
   const dvec2_t* b2 = reinterpret_cast<const dvec2_t*>(base) + local;
+  M[17] = M[23] = M[25] = M[26] = 0;  // not kept, not used
 #pragma unroll
-  for (int j = 0; j < 13; j++) {
+  for (int j = 0; j < kMom3 / 2; j++) {
     const dvec2_t v = ld_mom<NT>(b2 + j * kTileThreads);
-    M[2 * j] = v.x;
-    M[2 * j + 1] = v.y;
+    M[mom_of_slot(2 * j)] = v.x;
+    M[mom_of_slot(2 * j + 1)] = v.y;
   }
-  M[26] = ld_mom<NT>(base + 26 * kTileThreads + local);
+  M[mom_of_slot(kMom3 - 1)] = ld_mom<NT>(base + (kMom3 - 1) * kTileThreads + local);
 }
 template <bool NT>
 __device__ __forceinline__ void load_tile_moments3(const float* __restrict__ Mom, long long tile, int local,
                                                    float (&M)[27]) {
-  const float* base = Mom + tile * 27 * kTileThreads;
+  const float* base = Mom + tile * kMom3 * kTileThreads;
   const fvec4_t* b4 = reinterpret_cast<const fvec4_t*>(base) + local;
+  M[17] = M[23] = M[25] = M[26] = 0;
 #pragma unroll
-  for (int j = 0; j < 6; j++) {
+  for (int j = 0; j < kMom3 / 4; j++) {
     const fvec4_t v = ld_mom<NT>(b4 + j * kTileThreads);
-    M[4 * j] = v.x;
-    M[4 * j + 1] = v.y;
-    M[4 * j + 2] = v.z;
-    M[4 * j + 3] = v.w;
+    M[mom_of_slot(4 * j)] = v.x;
+    M[mom_of_slot(4 * j + 1)] = v.y;
+    M[mom_of_slot(4 * j + 2)] = v.z;
+    M[mom_of_slot(4 * j + 3)] = v.w;
   }
 #pragma unroll
-  for (int k = 24; k < 27; k++) M[k] = ld_mom<NT>(base + k * kTileThreads + local);
+  for (int q = kMom3 / 4 * 4; q < kMom3; q++) M[mom_of_slot(q)] = ld_mom<NT>(base + q * kTileThreads + local);
 }
 
-// The 27 moments of the element at lattice place (gi, gj, gk).
+// The moments of the element at lattice place (gi, gj, gk).
 template <typename T>
 __device__ __forceinline__ void load_moments3(const Geo& g, const T* __restrict__ Mom, int gi, int gj, int gk,
                                               T (&M)[27]) {
