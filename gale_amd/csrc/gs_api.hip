@@ -170,7 +170,7 @@ struct MGData {
   int* pos = nullptr;  // row of each dof of the coarsest level in the dense inverse, -1: Dirichlet
   double* Kinv64 = nullptr;
   float* Kinv32 = nullptr;
-  double* dwork = nullptr;    // inversion scratch
+  double* dwork = nullptr;    // scratch of the inversion and of the dense solve
   double* pow_d = nullptr;    // per level {lambda, scale, stopped} of the power iteration, then the pivot flag
   double* pow_h = nullptr;    // pinned copy
 };
@@ -1514,7 +1514,7 @@ static T* vcycle(gs_solver* s, int l, const T* b0 = nullptr, T* out = nullptr) {
     if (mg.nfc > 0) {
       T* x = out ? out : P.x;
       launch_dense_solve<T>(sizeof(T) == 8 ? (const T*)(void*)mg.Kinv64 : (const T*)(void*)mg.Kinv32, mg.freeidx,
-                            mg.pos, mg.nfc, mg.ldk, b, x, L.n, st);
+                            mg.pos, mg.nfc, mg.ldk, mg.dwork, b, x, L.n, st);
       return x;
     }
     return cheb_smooth<T>(L, 8, (T*)nullptr, st, b, out, &beta0);

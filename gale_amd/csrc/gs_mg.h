@@ -29,11 +29,18 @@ void launch_cheb(const T* b, const T* Ax, const T* dinv, T* d, T* x, long long n
 template <typename T>
 void launch_stencil_epi(const Geo& g, const T* A, const T* x, const TileEpi<T>& ep, hipStream_t st);
 // Dense coarsest solve x = Kinv b on the free dofs (nf at most
-// kDenseWideMax, rows of ld values), zero on the others (pos < 0).
+// kDenseWideMax, rows of ld values), zero on the others (pos < 0).  work: the
+// inversion's scratch (ld^2 / 64 values at most are used).
 constexpr int kDenseWideMax = 8192;
+// From this size of the inverse on, half of it is read, in two launches.
+// Measured, both launches against the one that reads all of it: n = 5577,
+// FP64 (249 MB) 27.3 against 48.0 us, FP32 (124 MB) 18.7 against 23.1 us;
+// n = 3267, FP64 (85 MB) 16.6 against 16.6 us; n = 1701, FP64 (23 MB) 10.1
+// against 9.0 us, FP32 9.6 against 6.4 us.
+constexpr long long kDenseSymBytes = 96LL << 20;
 template <typename T>
-void launch_dense_solve(const T* Kinv, const int* freeidx, const int* pos, int nf, int ld, const T* b, T* x,
-                        long long n, hipStream_t st);
+void launch_dense_solve(const T* Kinv, const int* freeidx, const int* pos, int nf, int ld, double* work, const T* b,
+                        T* x, long long n, hipStream_t st);
 // Power iteration on D^-1 K (x, Ax, d: n values); st4 in the level's slots.
 void launch_pow_init(double* x, const uint8_t* bc, long long n, double* st4, hipStream_t st);
 void launch_pow_step(double* x, const double* Ax, const double* dinv, double* d, long long n, double* st4, Reducer rd,

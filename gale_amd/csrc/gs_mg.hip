@@ -547,15 +547,111 @@ __global__ __launch_bounds__(1024) void k_dense_solve_wide(const T* __restrict__
   if (lane == 0) x[freeidx[row]] = s;
 }
 
+// Kinv is symmetric, so a solve can read half of it: a wave takes one 64 x 64
+// tile (i, j), j <= i, of the lower triangle and adds both its row sums
+// (A x_j) and its column sums (A^T x_i).  Lane l holds the rows l / 8 + 8 k
+// and 64 / 8 columns of them, all 16-byte loads of a wave's tile in flight
+// together, and a sum goes over eight lanes only.  Slot s of P (nb slots of
+// ld values) holds what tile (s, .) or (., s) adds to a row, so every value is
+// written once and k_dense_sym_sum adds the slots in order.
+template <typename T, int M>
+__device__ __forceinline__ T sum8(T (&v)[8], int lane) {
+  // on return: the sum over the lanes that differ in bits M, 2M, 4M of v[i],
+  // i the three bits (4M: 4, 2M: 2, M: 1) of this lane
+#pragma unroll
+  for (int h = 4; h > 0; h >>= 1) {
+    const bool up = (lane & (h * M)) != 0;
+#pragma unroll
+    for (int a = 0; a < h; a++) {
+      const T send = up ? v[a] : v[a + h], keep = up ? v[a + h] : v[a];
+      v[a] = keep + __shfl_xor(send, h * M, 64);
+    }
+  }
+  return v[0];
+}
 template <typename T>
-void launch_dense_solve(const T* Kinv, const int* freeidx, const int* pos, int nf, int ld, const T* b, T* x,
-                        long long n, hipStream_t st) {
+__global__ __launch_bounds__(256) void k_dense_sym(const T* __restrict__ Kinv, int ld, int ntile,
+                                                   const int* __restrict__ freeidx, int nf, const T* __restrict__ b,
+                                                   T* __restrict__ P) {
+  constexpr int E = 16 / (int)sizeof(T), Q = 64 / (8 * E);
+  typedef T vec_t __attribute__((ext_vector_type(E)));
+  __shared__ T sx[4][128];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int t = blockIdx.x * 4 + w;
+  const bool live = t < ntile;
+  int i = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
+  while ((i + 1) * (i + 2) / 2 <= t) i++;
+  while (i * (i + 1) / 2 > t) i--;
+  const int j = t - i * (i + 1) / 2;
+  const int lr = lane >> 3, lc = lane & 7;
+  vec_t v[8][Q];
+  if (live) {
+    const T* base = Kinv + ((long long)i * 64 + lr) * ld + j * 64 + lc * E;
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+#pragma unroll
+      for (int q = 0; q < Q; q++) v[k][q] = *reinterpret_cast<const vec_t*>(base + (long long)8 * k * ld + q * 8 * E);
+    const int r = i * 64 + lane, c = j * 64 + lane;
+    sx[w][lane] = r < nf ? b[freeidx[r]] : T(0);
+    sx[w][64 + lane] = c < nf ? b[freeidx[c]] : T(0);
+  }
+  __syncthreads();
+  if (!live) return;
+  T rs[8], cs[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) rs[k] = cs[k] = 0;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const T xr = sx[w][8 * k + lr];
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+#pragma unroll
+      for (int e = 0; e < E; e++) {
+        rs[k] += v[k][q][e] * sx[w][64 + (q * 8 + lc) * E + e];
+        cs[q * E + e] += v[k][q][e] * xr;
+      }
+  }
+  const T rsum = sum8<T, 1>(rs, lane), csum = sum8<T, 8>(cs, lane);
+  P[(long long)j * ld + i * 64 + 8 * lc + lr] = rsum;
+  if (i != j) P[(long long)i * ld + j * 64 + (lr / E * 8 + lc) * E + lr % E] = csum;
+}
+template <typename T>
+__global__ __launch_bounds__(256) void k_dense_sym_sum(const T* __restrict__ P, int ld, const int* __restrict__ freeidx,
+                                                       const int* __restrict__ pos, int nf, T* __restrict__ x,
+                                                       long long n) {
+  __shared__ T part[8][32];
+  const int c = threadIdx.x & 31, g = threadIdx.x >> 5, nb = ld / 64;
+  const int e = blockIdx.x * 32 + c;
+  T s = 0;
+#pragma unroll 8
+  for (int k = g; k < nb; k += 8) s += P[(long long)k * ld + e];
+  part[g][c] = s;
+  for (long long q = blockIdx.x * 256LL + threadIdx.x; q < n; q += (long long)gridDim.x * 256)
+    if (pos[q] < 0) x[q] = 0;
+  __syncthreads();
+  if (g == 0 && e < nf) {
+#pragma unroll
+    for (int k = 1; k < 8; k++) s += part[k][c];
+    x[freeidx[e]] = s;
+  }
+}
+
+template <typename T>
+void launch_dense_solve(const T* Kinv, const int* freeidx, const int* pos, int nf, int ld, double* work, const T* b,
+                        T* x, long long n, hipStream_t st) {
+  if ((long long)nf * nf * (long long)sizeof(T) >= kDenseSymBytes) {
+    const int nb = ld / 64, ntile = nb * (nb + 1) / 2;
+    T* P = reinterpret_cast<T*>(work);
+    hipLaunchKernelGGL(k_dense_sym<T>, dim3((ntile + 3) / 4), dim3(256), 0, st, Kinv, ld, ntile, freeidx, nf, b, P);
+    hipLaunchKernelGGL(k_dense_sym_sum<T>, dim3(ld / 32), dim3(256), 0, st, P, ld, freeidx, pos, nf, x, n);
+    return;
+  }
   hipLaunchKernelGGL(k_dense_solve_wide<T>, dim3(nf > 0 ? (nf + 15) / 16 : 1), dim3(1024), 0, st, Kinv, ld, freeidx,
                      pos, nf, b, x, n);
 }
-template void launch_dense_solve<double>(const double*, const int*, const int*, int, int, const double*, double*,
-                                         long long, hipStream_t);
-template void launch_dense_solve<float>(const float*, const int*, const int*, int, int, const float*, float*,
+template void launch_dense_solve<double>(const double*, const int*, const int*, int, int, double*, const double*,
+                                         double*, long long, hipStream_t);
+template void launch_dense_solve<float>(const float*, const int*, const int*, int, int, double*, const float*, float*,
                                         long long, hipStream_t);
 
 // Power iteration on D^-1 K: x = 1 on the free dofs, then per step
