@@ -304,59 +304,80 @@ __global__ __launch_bounds__(256) void k_conv_tiled(const uint16_t* __restrict__
   const long long b = t / tz;
   const int x0 = bx * 16, y0 = by * 4, z0 = bz * 4;
   const long long bbase = b * (long long)nx * ny * nz;
-  if constexpr (Q % 2 == 0) {
-    // 16-byte pieces (8 channels) when a voxel holds a whole number of them
-    constexpr int Q8 = Q / 2;
-    const s8* in8 = reinterpret_cast<const s8*>(in);
-    s8* box8 = reinterpret_cast<s8*>(box);
-    for (int q = threadIdx.x; q < NBOX * Q8; q += 256) {
-      const int c8 = q % Q8, vx = q / Q8;
-      const int xx = vx % BX, yy = (vx / BX) % BY, zz = vx / (BX * BY);
-      const int gx = x0 - 1 + xx, gy = y0 - 1 + yy, gz = z0 - 1 + zz;
-      s8 v = s8{0, 0, 0, 0, 0, 0, 0, 0};
-      if (gx >= 0 && gx < nx && gy >= 0 && gy < ny && gz >= 0 && gz < nz)
-        v = in8[(bbase + gx + (long long)nx * (gy + (long long)ny * gz)) * Q8 + c8];
-      box8[q] = v;
-    }
-  } else {
-    const s4* in4 = reinterpret_cast<const s4*>(in);
-    for (int q = threadIdx.x; q < NBOX * Q; q += 256) {
-      const int c4 = q % Q, vx = q / Q;
-      const int xx = vx % BX, yy = (vx / BX) % BY, zz = vx / (BX * BY);
-      const int gx = x0 - 1 + xx, gy = y0 - 1 + yy, gz = z0 - 1 + zz;
-      s4 v = s4{0, 0, 0, 0};
-      if (gx >= 0 && gx < nx && gy >= 0 && gy < ny && gz >= 0 && gz < nz)
-        v = in4[(bbase + gx + (long long)nx * (gy + (long long)ny * gz)) * Q + c4];
-      box[q] = v;
-    }
+  // A thread's pieces of the box are all requested before the first is
+  // written to LDS, and the first weights before the barrier; the K loop is
+  // unrolled, so that a step's place in the box costs at most three selects
+  // instead of divisions.  16 to 16 channels at 96^3: 30.2 -> 25.4 us, the
+  // network there 342 -> 315 us (57 MB in and out: 11 us at the copy rate).
+  constexpr int PS = Q % 2 == 0 ? 8 : 4;  // channels of a piece: 16 bytes where a voxel holds a whole number of them
+  typedef short piece_t __attribute__((ext_vector_type(PS)));
+  constexpr int QP = CIN / PS, NP = (NBOX * QP + 255) / 256;
+  const piece_t* inp = reinterpret_cast<const piece_t*>(in);
+  piece_t* boxp = reinterpret_cast<piece_t*>(box);
+  piece_t pv[NP];
+  bool pin[NP];
+#pragma unroll
+  for (int i = 0; i < NP; i++) {
+    const int q = threadIdx.x + 256 * i;
+    const int c = q % QP, vx = q / QP;
+    const int xx = vx % BX, yy = (vx / BX) % BY, zz = vx / (BX * BY);
+    const int gx = x0 - 1 + xx, gy = y0 - 1 + yy, gz = z0 - 1 + zz;
+    pin[i] = vx < NBOX && gx >= 0 && gx < nx && gy >= 0 && gy < ny && gz >= 0 && gz < nz;
+    pv[i] = inp[pin[i] ? (bbase + gx + (long long)nx * (gy + (long long)ny * gz)) * QP + c : 0];
   }
-  __syncthreads();
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int row = lane & 15, kg = lane >> 4;
+  // K steps in batches of U, the next batch's weights in flight
+  constexpr int U = NT == 1 ? 9 : (NT == 2 ? 5 : 3), NBATCH = (KC + U - 1) / U;
+  AT wv[2][U][NT];
+  auto load_w = [&](int n) {
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int v = 0; v < NT; v++)
+        if (n * U + u < KC) wv[n & 1][u][v] = Wp[((n * U + u) * NT + v) * 64 + lane];
+  };
+  load_w(0);
+#pragma unroll
+  for (int i = 0; i < NP; i++) {
+    const int q = threadIdx.x + 256 * i;
+    if (q < NBOX * QP) boxp[q] = pin[i] ? pv[i] : piece_t{};
+  }
+  __syncthreads();
   f4 acc[4][NT];
 #pragma unroll
   for (int j = 0; j < 4; j++)
 #pragma unroll
     for (int u = 0; u < NT; u++) acc[j][u] = f4{0.f, 0.f, 0.f, 0.f};
-  constexpr int U = 9;
-  for (int kc0 = 0; kc0 < KC; kc0 += U) {
-    AT wv[U][NT];
+  constexpr bool kOneTap = CIN % KW == 0;  // a K step lies in one tap
+  const s4* bw = box + (w * BY * BX + row) * Q + (kOneTap ? kg * (KW / 16) : 0);
 #pragma unroll
-    for (int u = 0; u < U; u++)
-#pragma unroll
-      for (int v = 0; v < NT; v++) wv[u][v] = kc0 + u < KC ? Wp[((kc0 + u) * NT + v) * 64 + lane] : AT{};
+  for (int n = 0; n < NBATCH; n++) {
+    if (n + 1 < NBATCH) load_w(n + 1);
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const int kk = (kc0 + u) * KW + kg * (KW / 4);  // this lane's first K index of the step
-      const bool in_k = kc0 + u < KC && kk < KT;
-      const int tap = kk / CIN, ci = kk - tap * CIN;
-      const int dx = tap % 3, dy = (tap / 3) % 3, dz = tap / 9;
+      const int kc = n * U + u;
+      if (kc >= KC) break;
+      // this lane's first K index of the step is kc KW + kg KW / 4: its place
+      // in the box is one of four constants (linear in kg within a tap)
+      auto place = [&](int g) {
+        const int kk = kc * KW + g * (KW / 4), tap = kk / CIN;
+        return ((tap / 9 * BY + tap / 3 % 3) * BX + tap % 3) * Q + (kk - tap * CIN) / 4;
+      };
+      auto in_k = [&](int g) { return kc * KW + g * (KW / 4) < KT; };
+      int o = place(0);
+      bool ok = true;
+#pragma unroll
+      for (int g = 1; g < (kOneTap ? 1 : 4); g++) {
+        if (in_k(g)) o = kg >= g ? place(g) : o;
+        if (!in_k(g)) ok = ok && kg != g;
+      }
 #pragma unroll
       for (int j = 0; j < 4; j++) {
-        const AT a = in_k ? *reinterpret_cast<const AT*>(&box[(((w + dz) * BY + (j + dy)) * BX + (row + dx)) * Q + ci / 4])
-                          : AT{};
+        AT a = *reinterpret_cast<const AT*>(bw + o + j * BX * Q);
+        if (!ok) a = AT{};
 #pragma unroll
-        for (int v = 0; v < NT; v++) acc[j][v] = mfma_bf16(a, wv[u][v], acc[j][v]);
+        for (int v = 0; v < NT; v++) acc[j][v] = mfma_bf16(a, wv[n & 1][u][v], acc[j][v]);
       }
     }
   }
