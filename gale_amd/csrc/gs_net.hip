@@ -517,13 +517,16 @@ __global__ void k_bgrad_reduce(const float* __restrict__ bpart, int n, int C, fl
 // P[group][(tap * cin + ci)][co] over the group's share of the voxels: block
 // (m tile, dy, dz) x group, its four waves a quarter of the group each, three
 // taps (dx) x NT column tiles of 16x16 accumulators a wave.  Per 32-voxel K
-// step a wave issues 3 + NT 16-byte loads for 3 NT v_mfma_f32_16x16x32_bf16,
-// the next step's in flight.  For eight 32^3 samples (the padded 16-channel
-// level is 10 MB) the 16-channel layers take 111 us, bound by the half cache
-// lines that 16 rows of 64 bytes fetch from L2, where gathering operands in
-// 2-byte loads from the channels-last tensors took 355 us; the whole backward
-// 2.4 ms (6.2 before, with the bias sums below).
-typedef s8 s8u __attribute__((aligned(2)));  // a tap's shift leaves 2-byte alignment
+// step a wave loads a row's eight values with the dwords before and after
+// them and NT 16-byte pieces of G for 3 NT v_mfma_f32_16x16x32_bf16, the next
+// step's in flight; the taps dx = -1, 1 are those values shifted by 16 bits.
+// Loading each tap instead (16 bytes from an odd element) was what bounded
+// the kernel: for eight 32^3 samples the 16-channel layers took 110 us and
+// now take 38, the 32-channel ones 29 and 14.  Neither whole 128-byte lines
+// per row nor keeping the nine blocks of a group on one XCD changed it.
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
+typedef u4 u4u __attribute__((aligned(2)));  // a tap's shift leaves 4-byte alignment, 2-byte on a grid of odd width
+typedef unsigned u1u __attribute__((aligned(2)));
 template <int NT>
 __global__ __launch_bounds__(256) void k_wgrad(const uint16_t* __restrict__ X, const uint16_t* __restrict__ G,
                                                long long stride, int cin, int cout, int w, int pl, long long kper,
@@ -542,18 +545,29 @@ __global__ __launch_bounds__(256) void k_wgrad(const uint16_t* __restrict__ X, c
   for (int q = 0; q < 3; q++)
 #pragma unroll
     for (int t = 0; t < NT; t++) acc[q][t] = f4{0.f, 0.f, 0.f, 0.f};
-  s8 a[3], g[NT];
+  // the eight values of the middle tap and the dwords before and after them
+  u4 a;
+  unsigned al, ar;
+  s8 g[NT];
   auto load = [&](long long k) {
-#pragma unroll
-    for (int q = 0; q < 3; q++) a[q] = *reinterpret_cast<const s8u*>(xa + k + (q - 1));
+    a = *reinterpret_cast<const u4u*>(xa + k);
+    al = *reinterpret_cast<const u1u*>(xa + k - 2);
+    ar = *reinterpret_cast<const u1u*>(xa + k + 8);
 #pragma unroll
     for (int t = 0; t < NT; t++) g[t] = *reinterpret_cast<const s8*>(gb + (long long)t * 16 * stride + k);
   };
   if (k0 < k1) load(k0);
   for (long long k = k0; k < k1; k += 32) {
     s8 ac[3], gc[NT];
+    u4 lo, hi;  // the values shifted by one voxel either way
 #pragma unroll
-    for (int q = 0; q < 3; q++) ac[q] = a[q];
+    for (int i = 0; i < 4; i++) {
+      lo[i] = __builtin_amdgcn_alignbit(a[i], i ? a[i ? i - 1 : 0] : al, 16);
+      hi[i] = __builtin_amdgcn_alignbit(i < 3 ? a[i < 3 ? i + 1 : 3] : ar, a[i], 16);
+    }
+    ac[0] = __builtin_bit_cast(s8, lo);
+    ac[1] = __builtin_bit_cast(s8, a);
+    ac[2] = __builtin_bit_cast(s8, hi);
 #pragma unroll
     for (int t = 0; t < NT; t++) gc[t] = g[t];
     if (k + 32 < k1) load(k + 32);
