@@ -1158,11 +1158,13 @@ static BArgs make_args(gs_batch* b, const gs_batch_params* p) {
 }
 
 // Direction rings of the relaxed loop (allocated on first use, before any
-// graph capture).
+// graph capture).  A captured graph holds their addresses, so it goes with the
+// rings it was captured with.
 static int32_t ensure_rings(gs_batch* b, const gs_batch_params* p) {
   if (!(p->inner_relax_max > 0)) return GS_OK;
   const int m = p->flexible_window > 0 ? std::min(p->flexible_window, kBatchMaxWin) : 8;
   if (b->fs && b->fwin == m) return GS_OK;
+  free_graph(b);
   if (b->fs) (void)hipFree(b->fs);
   if (b->fq) (void)hipFree(b->fq);
   b->fs = b->fq = nullptr;
