@@ -176,6 +176,13 @@ struct MGData {
 };
 constexpr int kMaxLevels = 17;
 
+// Free dofs of the coarsest level up to which a batch takes its inverse.  A
+// mesh that does not coarsen has no other level, and its inverse rounded to
+// FP32 is then the whole preconditioner: 4 inner iterations a solve at a
+// viscosity contrast of 1e4, about 23 at 1e6 (13 x 40 and 31 x 31), none that
+// converge at 1e7.
+constexpr int kBatchDenseMax = 2000;
+
 static void mg_free(MGData& mg);
 
 struct gs_solver {
@@ -1254,8 +1261,8 @@ static int32_t mg_structure(gs_solver* s) {
   // dense).  The batched solver runs each instance's coarsest solve inside
   // one workgroup, which reads the inverse from L2 at one compute unit's
   // rate: there it stops at 200 free dofs (10^2 with free-slip walls, 0.16
-  // MB), below at least one smoothed level (its V-cycle is FP32 throughout);
-  // 32 sinkers of 16^2 to 48^2, four seeds: 794 ms against 954 with levels
+  // MB), below at least one smoothed level wherever the mesh coarsens (its
+  // V-cycle is FP32 throughout); 32 sinkers of 16^2 to 48^2, four seeds: 794 ms against 954 with levels
   // down to 2 elements a side.  300 dofs (12^2) take 631 ms, but there the
   // solution of a 24^2 instance was twice as far from the converged one.
   // GALE_MG_DENSE_STOP=0 / 1 overrides (A/B timing).
@@ -1618,7 +1625,7 @@ void gs::batch_mark(gs_solver* s) { s->for_batch = true; }
 int32_t gs::batch_mg_info(gs_solver* s, int* nlev, BatchLevelInfo* lv, int max_levels, int* nfc) {
   if (!s || !s->setup_done || !s->mg.structured || s->pb->dim != 2) return GS_E_INVALID;
   const int n = s->mg.L + 1;
-  if (n > max_levels) return GS_E_INVALID;
+  if (n > max_levels || s->mg.nfc > kBatchDenseMax) return GS_E_INVALID;
   for (int l = 0; l < n; l++) lv[l] = BatchLevelInfo{s->mg.lv[l].g.res[0], s->mg.lv[l].g.res[1], s->mg.lv[l].lmax};
   *nlev = n;
   *nfc = s->mg.nfc;

@@ -56,7 +56,10 @@ typedef struct gs_batch_result {
   double seconds;            /* device time the instance's solve took inside the launch */
 } gs_batch_result;
 
-/* count problem descriptions (2D); each instance is set up on the device. */
+/* count problem descriptions (2D); each instance is set up on the device.
+ * Refused (GS_E_INVALID) when an instance's coarsest level (the mesh with its
+ * axes halved while both are even) has 2001 to 6000 free dofs: its inverse
+ * would be the only level of a mesh that does not coarsen, in FP32. */
 int32_t gs_batch_create(int32_t count, const gs_problem_desc* descs, gs_batch** out);
 void gs_batch_destroy(gs_batch* b);
 /* Workgroup shape of the batched solve: block in {256, 512, 1024} threads,
