@@ -164,8 +164,10 @@ struct MGData {
   int L = 0;  // index of the coarsest level
   std::vector<MGLevel> lv;
   int nfc = 0;
-  int ldk = 0;         // row length of the dense inverse (ldk x ldk, padding the identity)
-  int dense_from = 0;  // first level whose dense inverse may be taken (raised when one is not positive definite)
+  int ldk = 0;           // row length of the dense inverse (ldk x ldk, padding the identity)
+  int dense_from = 0;    // first level whose dense inverse may be taken (raised when one is not positive definite)
+  bool deepest = false;  // coarsening ended where the mesh or its flags do not allow more
+  bool failed = false;   // the last setup found no level with a dense inverse: nothing to precondition with
   int* freeidx = nullptr;
   int* pos = nullptr;  // row of each dof of the coarsest level in the dense inverse, -1: Dirichlet
   double* Kinv64 = nullptr;
@@ -1271,13 +1273,17 @@ static int32_t mg_structure(gs_solver* s) {
   const int dense_max = dense_max_free();
   const int stop_max = s->for_batch ? 200 : dense_max;
   const int stop_from = s->for_batch ? std::max(1, mg.dense_from) : mg.dense_from;
+  mg.deepest = true;
   for (int lev = 0; lev < 16; lev++) {
     const Geo& gf = mg.lv.back().g;
     if (dense_stop && lev >= stop_from) {
       long long nfree = 0;
       for (long long n = 0; n < gf.N; n++)
         for (int d = 0; d < dim; d++) nfree += ((flag[n] >> d) & 1u) ? 0 : 1;
-      if (nfree <= stop_max) break;
+      if (nfree <= stop_max) {
+        mg.deepest = false;
+        break;
+      }
     }
     bool ok = true;
     for (int d = 0; d < dim; d++) ok = ok && gf.res[d] % 2 == 0 && gf.res[d] / 2 >= 2;
@@ -1363,8 +1369,9 @@ static int32_t mg_structure(gs_solver* s) {
 }
 
 // Per-setup numeric part: moments of every level, Jacobi diagonals, the
-// Chebyshev bounds (power iteration on D^-1 K) and the dense coarse inverse.
-static int32_t mg_numeric(gs_solver* s) {
+// Chebyshev bounds (power iteration on D^-1 K) and the dense coarse inverse;
+// *bad: the dense operator is not positive definite to rounding.
+static int32_t mg_levels(gs_solver* s, bool* bad) {
   gs_problem* pb = s->pb;
   hipStream_t st = pb->st;
   MGData& mg = s->mg;
@@ -1401,26 +1408,42 @@ static int32_t mg_numeric(gs_solver* s) {
       launch_stencil_build<double>(L.g, L.M64, L.bcflag, L.A64, st);
     }
   }
-  int* bad = reinterpret_cast<int*>(mg.pow_d + 4 * kMaxLevels);
+  int* pivot_flag = reinterpret_cast<int*>(mg.pow_d + 4 * kMaxLevels);
   if (mg.nfc > 0) {
     const MGLevel& C = mg.lv[mg.L];
     launch_dense_assemble(C.g, C.M64, mg.pos, mg.nfc, mg.ldk, mg.Kinv64, st);
-    launch_spd_inverse(mg.Kinv64, mg.Kinv32, mg.ldk, mg.dwork, bad, st);
+    launch_spd_inverse(mg.Kinv64, mg.Kinv32, mg.ldk, mg.dwork, pivot_flag, st);
   }
   CK(hipMemcpyAsync(mg.pow_h, mg.pow_d, sizeof(double) * (4 * kMaxLevels + 1), hipMemcpyDeviceToHost, st));
   CK(hipStreamSynchronize(st));
   for (int l = 0; l < mg.L || (l == mg.L && mg.nfc < 0); l++) mg.lv[l].lmax = mg.pow_h[4 * l];
   int hbad = 0;
   std::memcpy(&hbad, mg.pow_h + 4 * kMaxLevels, sizeof(int));
-  if (mg.nfc > 0 && hbad) {
-    // not positive definite to rounding on this level: the next coarser one
-    // is tried, down to the smallest the mesh allows
-    const int L = mg.L;
-    mg.dense_from = L + 1;
-    CKS(mg_structure(s));
-    return mg.L > L ? mg_numeric(s) : GS_E_NAN;
-  }
+  *bad = mg.nfc > 0 && hbad;
   return GS_OK;
+}
+
+// A dense level that is not positive definite makes way for the next coarser
+// one, down to the smallest the mesh allows; every setup starts from the first
+// again, so that one bad field does not keep a solver on a deeper hierarchy.
+static int32_t mg_numeric(gs_solver* s) {
+  MGData& mg = s->mg;
+  if (mg.dense_from > 0) {
+    mg.dense_from = 0;
+    mg.structured = false;
+  }
+  mg.failed = false;
+  for (;;) {
+    bool bad = false;
+    CKS(mg_levels(s, &bad));
+    if (!bad) return GS_OK;
+    if (mg.deepest) {
+      mg.failed = true;
+      return GS_E_NAN;
+    }
+    mg.dense_from = mg.L + 1;
+    mg.structured = false;
+  }
 }
 
 template <typename T>
@@ -1726,6 +1749,7 @@ static int32_t inner_solve_jacobi(gs_solver* s, const double* b, double* x, doub
 // |r| <= rtol |b| stay FP64.
 static int32_t inner_solve_mg(gs_solver* s, const double* b, double* x, double rtol, long long* its) {
   gs_problem* pb = s->pb;
+  if (s->mg.failed) return GS_E_NAN;
   hipStream_t st = pb->st;
   const long long n = s->n;
   MGLevel& L0 = s->mg.lv[0];
