@@ -100,6 +100,7 @@ struct gs_problem {
   bool min_one_particle = true;
   double* out_xw = nullptr;  // local coordinates and weights in caller order (particle read-back)
   long long out_n = 0;       // particles it holds
+  std::mutex out_mutex;      // read-backs of one problem by several threads share these buffers
   double* halo64 = nullptr;  // tiled K apply scratch (fine level)
   float* halo32 = nullptr;
   int wkind = GS_WEIGHTS_CONSTANT;  // integration weights of the material points
@@ -505,6 +506,7 @@ extern "C" int32_t gs_problem_particles(gs_problem* pb, double* coord, int32_t* 
   const long long P = pb->P, E = pb->g.E;
   const int dim = pb->dim;
   hipStream_t st = pb->st;
+  std::lock_guard<std::mutex> lock(pb->out_mutex);
   CK(hipStreamSynchronize(st));
   if (P == 0 || !(coord || owner || xi || weight)) return GS_OK;
   // the device puts the state in caller order (coordinates and owners through

@@ -168,7 +168,8 @@ void gs_problem_destroy(gs_problem* pb);
 /* out5 = {N nodes, E elements, P particles, dim, escaped particles} */
 int32_t gs_problem_info(const gs_problem* pb, int64_t* out5);
 /* Particle state in the caller's original particle order: coord (P*3),
- * owner (P, -1 = outside), xi (P*dim), weight (P).  Any pointer may be NULL. */
+ * owner (P, -1 = outside), xi (P*dim), weight (P).  Any pointer may be NULL.
+ * Several threads may read one problem at once. */
 int32_t gs_problem_particles(gs_problem* pb, double* coord, int32_t* owner, double* xi, double* weight);
 
 /* Stokes_SLE + Stokes_SLE_UzawaSolver: _DefaultNew/_AssignFromXML/_Build
