@@ -1350,7 +1350,6 @@ static int32_t mg_structure(gs_solver* s) {
     CK(dalloc(&mg.pos, C.n));
     CK(hipMemcpy(mg.pos, pos.data(), sizeof(int) * C.n, hipMemcpyHostToDevice));
     CK(dalloc(&mg.Kinv64, (long long)mg.ldk * mg.ldk));
-    CK(dalloc(&mg.Kinv32, (long long)mg.ldk * mg.ldk));
     CK(dalloc(&mg.dwork, dense_work_count(mg.ldk)));
   } else {
     mg.nfc = -1;  // no dense coarse solve: Chebyshev smoothing on the coarsest level
@@ -1413,8 +1412,12 @@ static int32_t mg_levels(gs_solver* s, bool* bad) {
   int* pivot_flag = reinterpret_cast<int*>(mg.pow_d + 4 * kMaxLevels);
   if (mg.nfc > 0) {
     const MGLevel& C = mg.lv[mg.L];
+    // the FP32 copy (145 MB at 6000 free dofs) only where an FP32 V-cycle
+    // reads it (mg_fp32), or a batch
+    const bool f32 = s->for_batch || (s->up.precision == GS_PREC_MIXED && mg.L > 0);
+    if (f32 && !mg.Kinv32) CK(dalloc(&mg.Kinv32, (long long)mg.ldk * mg.ldk));
     launch_dense_assemble(C.g, C.M64, mg.pos, mg.nfc, mg.ldk, mg.Kinv64, st);
-    launch_spd_inverse(mg.Kinv64, mg.Kinv32, mg.ldk, mg.dwork, pivot_flag, st);
+    launch_spd_inverse(mg.Kinv64, f32 ? mg.Kinv32 : nullptr, mg.ldk, mg.dwork, pivot_flag, st);
   }
   CK(hipMemcpyAsync(mg.pow_h, mg.pow_d, sizeof(double) * (4 * kMaxLevels + 1), hipMemcpyDeviceToHost, st));
   CK(hipStreamSynchronize(st));

@@ -18,7 +18,8 @@ inline long long dense_work_count(int ld) { return 2LL * ld * kDenseBlock + kDen
 // Padding rows are the identity.
 void launch_dense_assemble(const Geo& g, const double* Mom, const int* pos, int nf, int ld, double* A, hipStream_t st);
 
-// A <- A^-1 (SPD, ld x ld, lower triangle read) with an FP32 copy in Af.
+// A <- A^-1 (SPD, ld x ld, lower triangle read) with an FP32 copy in Af where
+// that is not null.
 // *bad is set to 1 when a pivot is not positive and is left alone otherwise.
 void launch_spd_inverse(double* A, float* Af, int ld, double* work, int* bad, hipStream_t st);
 

@@ -205,7 +205,8 @@ __global__ __launch_bounds__(256) void k_sweep_update(double* __restrict__ A, in
         C[(long long)(16 * x + 4 * q + (lane >> 4)) * ld + 16 * y + (lane & 15)] = acc[x][y][q];
 }
 
-// A <- -A from the lower triangle, both triangles, with an FP32 copy.
+// A <- -A from the lower triangle, both triangles, with an FP32 copy (Af null:
+// without).
 __global__ __launch_bounds__(256) void k_sweep_finish(double* __restrict__ A, float* __restrict__ Af, int ld) {
   __shared__ double sp[NB][NB + 1];
   const long long t = blockIdx.x;
@@ -220,10 +221,10 @@ __global__ __launch_bounds__(256) void k_sweep_finish(double* __restrict__ A, fl
     const int a = q >> 6, b = q & 63;
     const double v = i == j && a < b ? sp[b][a] : sp[a][b];
     A[lo + (long long)a * ld + b] = v;
-    Af[lo + (long long)a * ld + b] = (float)v;
+    if (Af) Af[lo + (long long)a * ld + b] = (float)v;
     if (i != j) {
       A[up + (long long)a * ld + b] = sp[b][a];
-      Af[up + (long long)a * ld + b] = (float)sp[b][a];
+      if (Af) Af[up + (long long)a * ld + b] = (float)sp[b][a];
     }
   }
 }
