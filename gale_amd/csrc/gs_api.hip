@@ -1386,17 +1386,7 @@ static int32_t mg_levels(gs_solver* s, bool* bad) {
     launch_make_dinv(L.diag, L.bcdof, L.dinv64, L.n, st);
     launch_d2f(L.dinv64, L.dinv32, L.n, st);
   }
-  // Chebyshev upper bound: 12 power iterations on D^-1 K, the normalisation
-  // on the device (one host read for all levels instead of one per iteration)
   launch_fill(mg.pow_d, 4 * kMaxLevels + 1, 0.0, st);
-  for (int l = 0; l < mg.L || (l == mg.L && mg.nfc < 0); l++) {
-    MGLevel& L = mg.lv[l];
-    launch_pow_init(L.x, L.bcdof, L.n, mg.pow_d + 4 * l, st);
-    for (int it = 0; it < 12; it++) {
-      launch_mom_apply<double>(L.g, L.x, L.Ax, L.M64, L.bcflag, L.h64, st);
-      launch_pow_step(L.x, L.Ax, L.dinv64, L.d, L.n, mg.pow_d + 4 * l, s->rd, st);
-    }
-  }
   // assembled rows of the small smoothed levels, in the V-cycle's precision
   for (int l = 0; l < mg.L || (l == mg.L && mg.nfc < 0); l++) {
     MGLevel& L = mg.lv[l];
@@ -1418,6 +1408,19 @@ static int32_t mg_levels(gs_solver* s, bool* bad) {
     if (f32 && !mg.Kinv32) CK(dalloc(&mg.Kinv32, (long long)mg.ldk * mg.ldk));
     launch_dense_assemble(C.g, C.M64, mg.pos, mg.nfc, mg.ldk, mg.Kinv64, st);
     launch_spd_inverse(mg.Kinv64, f32 ? mg.Kinv32 : nullptr, mg.ldk, mg.dwork, pivot_flag, st);
+  }
+  // Chebyshev upper bound: 12 power iterations on D^-1 K, the normalisation
+  // on the device (one host read for all levels instead of one per iteration).
+  // Last and from the coarsest level to the finest, so that the setup ends in
+  // the applies that a solve begins with: the first apply after a setup takes
+  // 120 us at 96^3 with its operands in cache, and took 188 after the inverse.
+  for (int l = mg.nfc < 0 ? mg.L : mg.L - 1; l >= 0; l--) {
+    MGLevel& L = mg.lv[l];
+    launch_pow_init(L.x, L.bcdof, L.n, mg.pow_d + 4 * l, st);
+    for (int it = 0; it < 12; it++) {
+      launch_mom_apply<double>(L.g, L.x, L.Ax, L.M64, L.bcflag, L.h64, st);
+      launch_pow_step(L.x, L.Ax, L.dinv64, L.d, L.n, mg.pow_d + 4 * l, s->rd, st);
+    }
   }
   CK(hipMemcpyAsync(mg.pow_h, mg.pow_d, sizeof(double) * (4 * kMaxLevels + 1), hipMemcpyDeviceToHost, st));
   CK(hipStreamSynchronize(st));
