@@ -1,10 +1,9 @@
 """The dense coarsest multigrid solve on the 12^3 level (5577 free dofs with
-free-slip walls): the inverse is formed on the device (Cholesky factor and
-inverse) and applied by the wide row kernel.  A 48^3 hierarchy stops there
-(48-24-12); with the bound lowered to 2000 free dofs it goes on to 6^3 and
-the host-formed packed inverse.  Both V-cycles must give the same converged
-solution, FP64 and mixed precision, and the exact 12^3 coarse solve must not
-need more inner iterations."""
+free-slip walls), whose inverse the symmetric sweep forms on the device.  A
+48^3 hierarchy stops there (48-24-12); with the bound lowered to 2000 free
+dofs it goes on to the 6^3 level, inverted the same way.  Both V-cycles must
+give the same converged solution, FP64 and mixed precision, and the exact 12^3
+coarse solve must not need more inner iterations."""
 import numpy as np
 import pytest
 
