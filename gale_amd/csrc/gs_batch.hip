@@ -71,7 +71,7 @@ struct BInst {
 
 struct BLevel {
   int nx, ny;
-  long long node_off, elem_off;  // into the flat level arrays
+  long long node_off;  // into the flat level arrays
   double hx, hy, lmax;
 };
 
@@ -885,7 +885,7 @@ struct gs_batch {
   BInst* inst = nullptr;
   BLevel* lev = nullptr;
   int* order = nullptr;
-  long long nodes = 0, elems = 0, lnodes = 0, lelems = 0, kinv_n = 0, free_n = 0;
+  long long elems = 0;
   double4* FS = nullptr;
   double *f = nullptr, *dinv = nullptr, *Qinv = nullptr;
   uint8_t* bc = nullptr;
@@ -989,7 +989,7 @@ extern "C" int32_t gs_batch_create(int32_t count, const gs_problem_desc* descs, 
   constexpr int kMaxLev = 16;
   std::vector<std::vector<BatchLevelInfo>> info(count, std::vector<BatchLevelInfo>(kMaxLev));
   b->hinst.resize(count);
-  long long no = 0, eo = 0, lno = 0, leo = 0, ko = 0, fo = 0;
+  long long no = 0, eo = 0, lno = 0, ko = 0, fo = 0;
   for (int i = 0; i < count; i++) {
     const gs_problem_desc& d = descs[i];
     int32_t s = gs_problem_create(&d, &pbs[i]);
@@ -1022,21 +1022,14 @@ extern "C" int32_t gs_batch_create(int32_t count, const gs_problem_desc* descs, 
       L.nx = info[i][l].nx;
       L.ny = info[i][l].ny;
       L.node_off = lno;
-      L.elem_off = leo;
       L.hx = (d.hi[0] - d.lo[0]) / L.nx;
       L.hy = (d.hi[1] - d.lo[1]) / L.ny;
       L.lmax = info[i][l].lmax;
       b->hlev.push_back(L);
       lno += (long long)(L.nx + 1) * (L.ny + 1);
-      leo += (long long)L.nx * L.ny;
     }
   }
-  b->nodes = no;
   b->elems = eo;
-  b->lnodes = lno;
-  b->lelems = leo;
-  b->kinv_n = ko;
-  b->free_n = fo;
   const long long N2 = 2 * no, L2 = 2 * lno;
   if (balloc(&b->inst, count) || balloc(&b->lev, (long long)b->hlev.size()) || balloc(&b->order, count) ||
       balloc(&b->FS, kStencil * no) || balloc(&b->f, N2) || balloc(&b->dinv, N2) || balloc(&b->Qinv, eo) ||

@@ -126,7 +126,6 @@ void launch_recip(const double* a, double* b, long long n, hipStream_t st);
 void launch_scale(double* y, const double* x, double a, long long n, hipStream_t st);  // y = a*x
 void launch_axpby(double* y, const double* x, double a, double b, long long n, hipStream_t st); // y = a x + b y
 void launch_add(double* y, const double* a, const double* b, long long n, hipStream_t st);  // y = a + b
-void launch_mul(const double* a, const double* b, double* c, long long n, hipStream_t st);  // c = a * b
 
 // Inner CG (Jacobi).
 void launch_cg_init(const double* b, const double* dinv, double* x, double* r, double* p, long long n,

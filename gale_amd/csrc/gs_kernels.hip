@@ -162,14 +162,6 @@ void launch_add(double* y, const double* a, const double* b, long long n, hipStr
   hipLaunchKernelGGL(k_add, dim3(grid_for(n)), dim3(kBlock), 0, st, y, a, b, n);
 }
 
-__global__ void k_mul(const double* __restrict__ a, const double* __restrict__ b, double* __restrict__ c, long long n) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-    c[i] = a[i] * b[i];
-}
-void launch_mul(const double* a, const double* b, double* c, long long n, hipStream_t st) {
-  hipLaunchKernelGGL(k_mul, dim3(grid_for(n)), dim3(kBlock), 0, st, a, b, c, n);
-}
-
 __global__ void k_dot(const double* __restrict__ a, const double* __restrict__ b, long long n, double* S, int slot,
                       Reducer rd) {
   double v[1] = {0.0};

@@ -57,6 +57,4 @@ void launch_pow_step(double* x, const double* Ax, const double* dinv, double* d,
 // 10.9 s in total.
 constexpr double kChebLow = 0.2, kChebHigh = 1.1;
 
-inline int n_moments(int dim) { return dim == 2 ? 9 : 27; }
-
 }  // namespace gs
