@@ -1258,6 +1258,10 @@ extern "C" int32_t gs_batch_autotune(gs_batch* b, const gs_batch_params* p, int3
   int best = b->tile;
   float best_ms = 1e30f;
   for (int k = 0; k < 6; k++) {
+    if (k > 0 && kTiles[k].bs == kTiles[k - 1].bs) {  // the same kernel
+      if (ms) ms[k] = ms[k - 1];
+      continue;
+    }
     BCK(hipEventRecord(b->e0, b->st));
     launch_batch(b, A, k, b->st);
     BCK(hipGetLastError());

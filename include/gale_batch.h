@@ -10,9 +10,9 @@
  * synchronisation is needed.  The inner velocity solve is FP64 flexible CG
  * preconditioned by one FP32 geometric-multigrid V-cycle (the instance's
  * Galerkin levels built by the single-problem setup; FP32 K applies, FP64
- * vectors, dots and outer loop).  The element-tile shape of the K apply
- * (workgroup size x tile width) is chosen by gs_batch_autotune; the solve can
- * be captured once as a HIP graph and replayed.
+ * vectors, dots and outer loop).  The workgroup size is chosen by
+ * gs_batch_autotune; the solve can be captured once as a HIP graph and
+ * replayed.
  *
  * Instances: 2D, homogeneous Dirichlet conditions (e.g. free slip), no
  * yielding (first, linear solve).  Setup of each instance (particle
@@ -66,9 +66,10 @@ void gs_batch_destroy(gs_batch* b);
  * tx in {16, 32, 64} (one of the shapes below; shapes of one block size run
  * alike, the stencil applies walk the nodes in order). */
 int32_t gs_batch_set_tile(gs_batch* b, int32_t block, int32_t tx);
-/* Times every shape on this batch (a few Uzawa iterations each, HIP
- * events) and keeps the fastest; ms receives one time per candidate in the
- * order (256,16) (256,32) (512,32) (512,64) (1024,32) (1024,64). */
+/* Times every block size on this batch (a few Uzawa iterations each, HIP
+ * events) and keeps the fastest, at its first tx; ms receives one time per
+ * candidate in the order (256,16) (256,32) (512,32) (512,64) (1024,32)
+ * (1024,64), the same for both shapes of a block size. */
 int32_t gs_batch_autotune(gs_batch* b, const gs_batch_params* p, int32_t* block, int32_t* tx, float* ms);
 /* Solves every instance (results: count entries, may be NULL); seconds = device
  * time of the launch. */

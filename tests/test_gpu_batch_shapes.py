@@ -39,3 +39,13 @@ def test_batch_branches(gale, block, tx, relax):
         us, ps, _ = s.Solve()
         assert rel(u, us) < 1e-7, (MESHES[i], rel(u, us))
         assert rel(p - p.mean(), ps - ps.mean()) < 1e-6, (MESHES[i], rel(p - p.mean(), ps - ps.mean()))
+
+
+def test_autotune_times_each_block_size_once(gale):
+    """The two widths of a block size are one kernel: one time for both, and
+    the fastest block size at its first width."""
+    bs = gale.BatchSolver([_problem(gale, nx, ny, i) for i, (nx, ny) in enumerate([(16, 16), (24, 24)])])
+    best, ms = bs.autotune(gale.batch_params(tolerance=1e-6))
+    t = [ms[c] for c in gale.TILE_CANDIDATES]
+    assert t[0] == t[1] and t[2] == t[3] and t[4] == t[5] and min(t) > 0
+    assert best == gale.TILE_CANDIDATES[t.index(min(t))]
