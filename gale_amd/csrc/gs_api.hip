@@ -138,9 +138,15 @@ struct MGLevel {
   float* A32 = nullptr;
 };
 
-// Levels whose assembled rows take at most this (in FP64: 33^3 nodes in 3D,
-// 500^2 in 2D) are smoothed from them; larger ones, whose rows would come from
-// HBM, from their moments (48^3 nodes: 228 MB against 24 MB).
+// Levels whose assembled rows take at most this, counted in FP64 (33^3 nodes
+// in 3D, 500^2 in 2D), are smoothed from them; larger ones, whose rows would
+// come from HBM, from their moments (48^3 elements: 229 MB against 20 MB).
+// Microseconds of an inner iteration with the finest level's rows against its
+// moments, the coarser levels assembled in both: FP64 24^3 107 / 142, 32^3 (70
+// MB) 137 / 155, 36^3 (98 MB) 164 / 165, 40^3 197 / 174, 48^3 306 / 212; 2D
+// 512^2 (76 MB) 197 / 214, 640^2 (118 MB) 262 / 256.  In mixed precision the
+// rows take half and would pay to about 45^3: 36^3 126 / 156, 40^3 146 / 163,
+// 48^3 190 / 180.
 constexpr long long kStencilBytes = 72LL << 20;
 static bool assembled_level(const Geo& g) { return stencil_count(g) * 8 <= kStencilBytes; }
 

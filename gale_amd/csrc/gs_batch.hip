@@ -377,9 +377,12 @@ struct Inst {
   double *fs, *fq;
 };
 
-// Chebyshev-Jacobi smoothing on one level (FP32), window [0.1, 1.1] lmax (in
-// 2D the lower bound makes no difference here): zero = start from x = 0.  x starts in `x`
-// (or in Lx when zero) and ping-pongs; returns the buffer that holds it.
+// Chebyshev-Jacobi smoothing on one level (FP32), window [0.1, 1.1] lmax: zero
+// = start from x = 0.  x starts in `x` (or in Lx when zero) and ping-pongs;
+// returns the buffer that holds it.  Sinkers of 16^2 to 48^2 take 1 to 4 %
+// fewer inner iterations from 0.2 lmax (the single solver's bound) and no less
+// time: 115 / 334 / 184 / 174 ms for four seeds' batches, 110 / 331 / 177 / 174
+// from 0.1.
 template <int BS>
 __device__ float* bsmooth(const BArgs& A, const BLevel& L, int nu, bool zero, float* x) {
   const int w = L.nx + 1, h = L.ny + 1, N = w * h;
@@ -904,9 +907,11 @@ struct gs_batch {
   double *fs = nullptr, *fq = nullptr;  // relaxed loop direction rings (window x elements)
   int fwin = 0;
   unsigned* queue = nullptr;
-  // index into kTiles: 512 threads, the most whose registers do not spill (32
-  // sinkers of 16^2 to 48^2, three seeds, coarsest level 12^2: 77 / 280 / 131 ms against 115 / 392 /
-  // 176 with 256 threads and 104 / 326 / 167 with 1024; at 128^2 as fast as 1024)
+  // index into kTiles: 512 threads, the most whose vector registers do not
+  // spill (217 scalar ones do, to lanes of vector registers).  32 sinkers of
+  // 16^2 to 48^2, four seeds, reference loop: 110 / 331 / 177 / 174 ms, against
+  // 146 / 443 / 240 / 228 with 256 threads and 127 / 376 / 202 / 201 with 1024;
+  // one of 128^2 148 ms, 216 and 146.
   int tile = 2;
   int ncu = 256;
   hipEvent_t e0 = nullptr, e1 = nullptr;
