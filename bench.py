@@ -45,8 +45,8 @@ def k_apply_bytes(dim, N, E, P, b=8):
 
 def k_moments_bytes(dim, N, E, b=8):
     """Algorithmic HBM bytes of one moment-form K apply: read u and write y,
-    and 27 (3D) / 9 (2D) moments per element."""
-    return 2 * b * dim * N + b * (27 if dim == 3 else 9) * E
+    and the 23 (3D) / 9 (2D) moments kept per element."""
+    return 2 * b * dim * N + b * (23 if dim == 3 else 9) * E
 
 
 def cpu_baseline(res, threads):
