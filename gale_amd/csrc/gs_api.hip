@@ -174,6 +174,7 @@ struct MGData {
   int ldk = 0;           // row length of the dense inverse (ldk x ldk, padding the identity)
   int dense_from = 0;    // first level whose dense inverse may be taken (raised when one is not positive definite)
   bool deepest = false;  // coarsening ended where the mesh or its flags do not allow more
+  bool current = false;  // the levels' moments are those of the solver's last setup
   bool failed = false;   // the last setup found no level with a dense inverse: nothing to precondition with
   int* freeidx = nullptr;
   int* pos = nullptr;  // row of each dof of the coarsest level in the dense inverse, -1: Dirichlet
@@ -1434,6 +1435,7 @@ static int32_t mg_levels(gs_solver* s, bool* bad) {
   int hbad = 0;
   std::memcpy(&hbad, mg.pow_h + 4 * kMaxLevels, sizeof(int));
   *bad = mg.nfc > 0 && hbad;
+  mg.current = true;
   return GS_OK;
 }
 
@@ -1629,6 +1631,7 @@ static int32_t setup_dev(gs_solver* s, const double* u_prev, const double* p_pre
   } else {
     launch_fill(s->h, s->np, 0.0, st);
   }
+  s->mg.current = false;
   if (s->up.inner_preconditioner == GS_INNER_MULTIGRID || s->up.precision == GS_PREC_MIXED) CKS(mg_numeric(s));
   if (s->lpc || s->rec) {
     if (!s->logeta) CK(dalloc(&s->logeta, s->np));
@@ -2355,10 +2358,8 @@ extern "C" int32_t gs_solver_sync(gs_solver* s) {
 
 extern "C" int32_t gs_apply_K_moments(gs_solver* s, const double* x, double* y) {
   if (!s || !x || !y) return GS_E_INVALID;
-  if (needs_setup(s) || !s->mg.structured) {
-    CKS(setup_dev(s, nullptr, nullptr, 0));
-    if (!s->mg.structured) CKS(mg_numeric(s));
-  }
+  if (needs_setup(s)) CKS(setup_dev(s, nullptr, nullptr, 0));
+  if (!s->mg.current) CKS(mg_numeric(s));
   launch_mom_apply<double>(s->mg.lv[0].g, x, y, s->mg.lv[0].M64, nullptr, s->mg.lv[0].h64, s->pb->st);
   s->k_applies++;
   return GS_OK;
@@ -2374,7 +2375,7 @@ extern "C" int32_t gs_time_apply(gs_solver* s, int32_t form, int32_t n_rep, int3
   gs_problem* pb = s->pb;
   hipStream_t st = pb->st;
   if (needs_setup(s)) CKS(setup_dev(s, nullptr, nullptr, 0));
-  if ((form == 2 || form == 3) && !s->mg.structured) CKS(mg_numeric(s));
+  if ((form == 2 || form == 3) && !s->mg.current) CKS(mg_numeric(s));
   if (form == 1) CKS(ensure_pk32(s));
   if (form == 1 || form == 3) {
     if (!s->x32) CK(dalloc(&s->x32, s->n));
