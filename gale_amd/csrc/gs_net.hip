@@ -1056,8 +1056,7 @@ static WgradPlan wgrad_plan(const Shape& sh, int l) {
 }
 static inline int wgrad_margin(const WgradPlan& p) { return p.pl + p.w + 2 + 32; }
 
-int ensure_work(Net* n, const Shape& sh) {
-  if (n->work.sh == sh && n->work.x4) return GS_OK;
+static int alloc_work(Net* n, const Shape& sh) {
   if (sh.nx % kGridMultiple || sh.ny % kGridMultiple || sh.nz % kGridMultiple || sh.nx < kGridMultiple ||
       sh.ny < kGridMultiple || sh.nz < kGridMultiple || sh.batch < 1)
     return GS_E_INVALID;
@@ -1108,6 +1107,18 @@ int ensure_work(Net* n, const Shape& sh) {
   NCK(hipMalloc(&w.bpart, sizeof(float) * bc));
   NCK(hipMalloc(&w.dpartial, sizeof(double) * 65536));
   return GS_OK;
+}
+
+// A shape that does not fit leaves nothing: with some of its buffers the next
+// call of that shape would take it for allocated.
+int ensure_work(Net* n, const Shape& sh) {
+  if (n->work.sh == sh && n->work.x4) return GS_OK;
+  const int e = alloc_work(n, sh);
+  if (e == GS_E_HIP) {
+    (void)hipGetLastError();
+    free_work(n->work);
+  }
+  return e;
 }
 
 // dispatch of the templated convolution kernels
